@@ -1,22 +1,34 @@
 // The SDF MLP of models/fields.py:85-99 (input_concat: h0 = [x, enc]; NH
 // hidden layers of width H with Softplus(beta, threshold 20); linear output of
-// width 1) as wavefront tiles on the fp32 matrix cores (v_mfma_f32_16x16x4f32).
+// width 1) in fp32 on the fp32 matrix cores (v_mfma_f32_16x16x4f32), the
+// activations in registers from layer to layer.
 //
-// A workgroup is 4 wavefronts; each wavefront owns a tile of T points (rows).
-// The tile's activations live in LDS (row-major, pitch padded by 4 floats);
-// the pre-folded (weight-normed) weights of every layer live in LDS for the
-// whole workgroup.  Each GEMM is a set of 16x16 output blocks, each the sum
-// over K in steps of 4 of one MFMA with strided LDS operand views
-//   A(i,k) = a[i*ai + k*ak],  B(k,j) = b[k*bk + j*bj],
-// so one helper serves Act*W^T (forward), G*W (backprop to the inputs) and
-// G^T*Act (weight gradients, K = the tile's points).
+// Layout.  Every layer is computed transposed, Z^T = W * H^T: units are the
+// MFMA rows and 16 points of a wavefront its columns.  With lane l, r = l % 16,
+// q = l / 16 one MFMA takes A[r][q], B[q][r] and returns D[4q + e][r], so a lane
+// ends a layer with point r's units 16 mb + 4q + e.  A dot product does not
+// depend on the order of K as long as A and B agree; the K axis of the next
+// layer is taken as step (mb, e), slot q -> unit 16 mb + 4q + e, which makes
+// the lane's own value (mb, e) its B operand, and the four weights of steps
+// (mb, 0..3) four consecutive floats of a weight row: one 16-byte LDS read per
+// four MFMAs (rows padded by 4 floats: conflict-free), no activation through
+// LDS.  The transposed products (W^T g of the backward) read the same weights
+// column-wise, one 4-byte read per MFMA.  h0 is held as [enc | x | 0 ...] in
+// KB blocks of 16 dims, so that a lane's four dims of a block are one 16-byte
+// load of the encoding.
 //
-// MFMA 16x16x4 fp32 lane mapping (lane l, r = l % 16, q = l / 16):
-//   A operand A[r][q], B operand B[q][r], result D[4q + e][r], e = 0..3.
+// Weight gradients need the points on the K axis: each step's gradient and
+// activation blocks go through two fp32 LDS tiles (64 rows x 64 points of a
+// workgroup's step) and back as 16-byte operands; the blocks are split over
+// the wavefronts.  Per-workgroup partial rows are summed in a fixed order by
+// mlp_reduce_rows, so results do not depend on scheduling (no float atomics).
 //
-// Weight gradients: each wavefront sums its tiles in registers in a fixed
-// order and writes one partial row; sn_mlp_reduce adds the rows in a fixed
-// order, so results do not depend on scheduling (no float atomics).
+// Bound: the fp32 matrix rate (32 cycles per MFMA and SIMD; 100 MFMAs per 16
+// points forward, ~330 backward at 35 -> 64 -> 64 -> 1) and the softplus VALU
+// work beside it.  Operands through LDS tiles with a wavefront per SIMD (the
+// weights and every activation in LDS) had measured 387 us forward and 560 us
+// backward over 299 593 points; 77 and 186 us with the activations in
+// registers.
 //
 // Packed parameter layout (fp32, row-major; the gradient uses the same):
 //   W0[H][d_in] b0[H] { W1[H][H] b1[H] } wo[H] bo
@@ -29,66 +41,77 @@ namespace sn {
 constexpr int kWaves = 4;
 constexpr float kSpThr = 20.f;
 
-__device__ __forceinline__ floatx4 mma_blk(const float* a, int ai, int ak, const float* b,
-                                           int bk, int bj, int K, floatx4 acc) {
-  const int l = threadIdx.x & 63, r = l & 15, q = l >> 4;
-#pragma unroll 4
-  for (int k = 0; k < K; k += 4)
-    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[r * ai + (k + q) * ak], b[(k + q) * bk + r * bj],
-                                               acc, 0, 0, 0);
-  return acc;
-}
-
-// Softplus(beta) with torch's threshold and its derivative e/(e+1), e = exp(beta z).
-__device__ __forceinline__ float sp(float z, float beta) {
-  const float bz = z * beta;
-  return bz > kSpThr ? z : log1pf(expf(bz)) / beta;
-}
-__device__ __forceinline__ float sp_d(float z, float beta) {
-  const float bz = z * beta;
-  if (bz > kSpThr) return 1.f;
-  const float e = expf(bz);
-  return e / (e + 1.f);
-}
-// d^2 softplus / dz^2 = beta s (1 - s) (0 above the threshold, where torch's
-// derivative is the constant 1).
-__device__ __forceinline__ float sp_dd(float z, float beta) {
-  const float bz = z * beta;
-  if (bz > kSpThr) return 0.f;
-  const float s = sp_d(z, beta);
-  return beta * s * (1.f - s);
-}
-
-__device__ __forceinline__ float sum16(float v) {  // over lanes with equal l / 16
-  v += __shfl_xor(v, 1, 64);
-  v += __shfl_xor(v, 2, 64);
-  v += __shfl_xor(v, 4, 64);
-  v += __shfl_xor(v, 8, 64);
-  return v;
-}
-__device__ __forceinline__ float sum4q(float v) {  // over lanes with equal l % 16
-  v += __shfl_xor(v, 16, 64);
-  v += __shfl_xor(v, 32, 64);
+// The lane's row and quarter, opaque to the compiler at each use: LDS
+// addresses derive from them and are formed where used; as loop invariants
+// they had been hoisted and held in ~80 registers.
+struct Lane {
+  int r, q;
+};
+__device__ __forceinline__ Lane lane_here() {
+  Lane v{(int)threadIdx.x & 15, ((int)threadIdx.x & 63) >> 4};
+  asm volatile("" : "+v"(v.r), "+v"(v.q));
   return v;
 }
 
-template <int H, int NH, int DP>
+__device__ __forceinline__ floatx4 mma(float a, float b, floatx4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+
+// Softplus(beta) with torch's threshold (z above it): value h, derivative
+// d = sigma(beta z) and its complement c = 1 - d (s'' = beta d c; 0 above the
+// threshold, where torch's derivative is the constant 1).  Branch-free, from
+// t = e^(-|beta z|) in (0, 1]: h = max(z, 0) + log1p(t) / beta (the large part
+// exact; log(1 + e^(beta z)) / beta from the hardware logarithm had a mean
+// error of -4e-8 in the sdf), d and c are 1 / (1 + t) and t / (1 + t).  On the
+// hardware exp2 / log2 / reciprocal, completed to about the accuracy of the
+// library functions: the low part of beta z log2(e) is multiplied back, log1p
+// takes the rounding of 1 + t as a correction, the reciprocal one Newton step.
+// A NaN z gives a NaN value.
+struct Sp {
+  float h, d, c;
+};
+template <bool kSecond = false>
+__device__ __forceinline__ Sp softplus(float z, float beta, float inv_beta) {
+  constexpr float kLog2e = 1.44269502f, kLog2eLo = 1.92596303e-8f, kLn2 = 0.693147182f;
+  const float bz = z * beta, a = -fabsf(bz);
+  const float p = a * kLog2e;
+  const float lo = fmaf(a, kLog2eLo, fmaf(a, kLog2e, -p)) * kLn2;
+  const float t0 = __builtin_amdgcn_exp2f(p);
+  const float t = fmaf(t0, lo, t0);
+  const float u = 1.f + t;
+  const float r0 = __builtin_amdgcn_rcpf(u);
+  const float r = fmaf(fmaf(-u, r0, 1.f), r0, r0);
+  const float tr = t * r;
+  const bool lin = bz > kSpThr, pos = bz >= 0.f;
+  Sp s;
+  const float l = fmaf(t - (u - 1.f), r, __builtin_amdgcn_logf(u) * kLn2) * inv_beta;
+  s.h = lin ? z : (pos ? z : 0.f) + l;
+  s.d = lin ? 1.f : (pos ? r : tr);
+  s.c = lin ? 0.f : (pos ? tr : r);
+  // selected here: sunk to their uses, the selections' masks are held instead
+  asm volatile("" : "+v"(s.h), "+v"(s.d));
+  if (kSecond) asm volatile("" : "+v"(s.c));
+  return s;
+}
+
+template <int H, int NH, int KB>
 struct Mlp {
-  static constexpr int LDI = DP + 4;
-  static constexpr int LDH = H + 4;
-  static constexpr int HB = H / 16;
-  static constexpr int IB = DP / 16;
-  // LDS weight offsets
-  static constexpr int oW0 = 0;
-  static constexpr int oB0 = oW0 + H * LDI;
-  static constexpr int oW1 = oB0 + H;
-  static constexpr int oB1 = oW1 + (NH == 2 ? H * LDH : 0);
-  static constexpr int oWo = oB1 + (NH == 2 ? H : 0);
-  static constexpr int oBo = oWo + H;
-  static constexpr int kWFloats = oBo + 4;
-  // per-wavefront buffers (floats per row)
-  static constexpr int kRow = LDI + 2 * LDH;
-  // global packed offsets
+  static constexpr int MB = H / 16;
+  static constexpr int D0 = 16 * KB;  // padded input dims
+  static constexpr int LD0 = D0 + 4, LD1 = H + 4;
+  // LDS (floats): weights, vectors b0 b1 wo bo, then the two block tiles
+  static constexpr int oW1 = H * LD0;
+  static constexpr int oVec = oW1 + (NH == 2 ? H * LD1 : 0);
+  static constexpr int kFwd = oVec + 3 * H + 4;
+  static constexpr int kRowsB = H > D0 ? H : D0;
+  static constexpr int kTileP = 16 * kWaves + 4;
+  static constexpr int oTA = kFwd, oTB = oTA + H * kTileP;
+  static constexpr int kBwd = oTB + kRowsB * kTileP;
+  // weight-gradient blocks: wavefront w owns column block w % MB of dW1 and
+  // row block w % MB of dW0, and every (kWaves / MB)-th of the other index
+  static constexpr int S = kWaves / MB;
+  static constexpr int T1 = NH == 2 ? MB / S : 1, T0 = (KB + S - 1) / S;
+  // packed parameter offsets
   __host__ __device__ static int n_params(int d) {
     return H * d + H + (NH == 2 ? H * H + H : 0) + H + 1;
   }
@@ -99,510 +122,603 @@ struct Mlp {
   __host__ __device__ static int gBo(int d) { return gWo(d) + H; }
 };
 
-template <int H, int NH, int DP>
-__device__ void load_weights(float* sw, const float* __restrict__ mlp, int d) {
-  using M = Mlp<H, NH, DP>;
-  for (int t = threadIdx.x; t < H * M::LDI; t += blockDim.x) {
-    const int o = t / M::LDI, i = t % M::LDI;
-    sw[M::oW0 + t] = (i < d) ? mlp[o * d + i] : 0.f;
-  }
-  for (int t = threadIdx.x; t < H; t += blockDim.x) {
-    sw[M::oB0 + t] = mlp[M::gB0(d) + t];
-    sw[M::oWo + t] = mlp[M::gWo(d) + t];
-    if (NH == 2) sw[M::oB1 + t] = mlp[M::gB1(d) + t];
+// packed W0 column of input dim c ([enc | x | pad]); -1 for padding
+__device__ __forceinline__ int in_col(int c, int E) {
+  return c < E ? 3 + c : (c < E + 3 ? c - E : -1);
+}
+
+template <int H, int NH, int KB>
+__device__ void load_weights(float* sw, const float* __restrict__ mlp, int E) {
+  using M = Mlp<H, NH, KB>;
+  const int d = 3 + E;
+  for (int t = threadIdx.x; t < H * M::LD0; t += blockDim.x) {
+    const int o = t / M::LD0, c = t % M::LD0;
+    const int col = c < M::D0 ? in_col(c, E) : -1;
+    sw[t] = col >= 0 ? mlp[o * d + col] : 0.f;
   }
   if (NH == 2)
-    for (int t = threadIdx.x; t < H * M::LDH; t += blockDim.x) {
-      const int o = t / M::LDH, i = t % M::LDH;
-      sw[M::oW1 + t] = (i < H) ? mlp[M::gW1(d) + o * H + i] : 0.f;
+    for (int t = threadIdx.x; t < H * M::LD1; t += blockDim.x) {
+      const int o = t / M::LD1, c = t % M::LD1;
+      sw[M::oW1 + t] = c < H ? mlp[M::gW1(d) + o * H + c] : 0.f;
     }
-  if (threadIdx.x == 0) sw[M::oBo] = mlp[M::gBo(d)];
+  float* vec = sw + M::oVec;
+  for (int t = threadIdx.x; t < H; t += blockDim.x) {
+    vec[t] = mlp[M::gB0(d) + t];
+    vec[H + t] = NH == 2 ? mlp[M::gB1(d) + t] : 0.f;
+    vec[2 * H + t] = mlp[M::gWo(d) + t];
+  }
+  if (threadIdx.x == 0) vec[3 * H] = mlp[M::gBo(d)];
 }
 
-// Rows [row0, row0+T) of [a3 | b] into an LDS tile (zero past n and past 3+E).
-template <int DP, int T>
-__device__ void load_rows(float* s, const float* __restrict__ a3, const float* __restrict__ b,
-                          int E, int64_t row0, int64_t n) {
-  constexpr int LDI = DP + 4;
-  const int lane = threadIdx.x & 63;
-  for (int t = lane; t < T * DP; t += 64) {
-    const int i = t / DP, c = t % DP;
-    const int64_t p = row0 + i;
-    float v = 0.f;
-    if (p < n) {
-      if (c < 3) v = a3[p * 3 + c];
-      else if (c < 3 + E) v = b[p * E + (c - 3)];
-    }
-    s[i * LDI + c] = v;
+// The 4 input dims 16 kb + 4q .. +3 of point p, zero past n and past E + 3.
+// With vec4 (E % 4 == 0, 16-byte rows) they are encoding dims (one load), the
+// position, or padding; otherwise one guarded load per dim.
+__device__ __forceinline__ void load_in(const float* __restrict__ x, const float* __restrict__ enc,
+                                        int E, int vec4, int64_t p, bool ok, int c4,
+                                        float (&v)[4]) {
+  if (vec4) {
+    float4 a = {0.f, 0.f, 0.f, 0.f};
+    if (ok && c4 < E) a = *reinterpret_cast<const float4*>(enc + p * E + c4);
+    else if (ok && c4 == E) a = float4{x[p * 3], x[p * 3 + 1], x[p * 3 + 2], 0.f};
+    v[0] = a.x;
+    v[1] = a.y;
+    v[2] = a.z;
+    v[3] = a.w;
+    return;
+  }
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int c = c4 + j;
+    const float* src = c < E ? enc + p * E + c : x + p * 3 + (c - E);
+    v[j] = 0.f;
+    if (ok && c < E + 3) v[j] = *src;
   }
 }
 
-// z = A*W^T (+ bias) for all (rb, cb) blocks of a tile.
-template <int T, int CB, bool kBias>
-__device__ __forceinline__ void gemm_xwT(const float* sA, int lda, const float* sW, int ldw,
-                                         const float* bias, int K, floatx4 (&z)[T / 16][CB]) {
-  const int r = (threadIdx.x & 63) & 15;
+// z[mb] += W (rows 16 mb + r) * b over NB blocks of 16 K dims.  (The scheduling
+// barriers keep the operand reads of one block from being hoisted over the
+// blocks before it: without them the backward kernels spilled up to 190
+// registers; the other wavefronts of the SIMD cover the reads.)
+template <int MB, int NB>
+__device__ __forceinline__ void gemm(const float* __restrict__ sw, int ld, const float (&b)[NB][4],
+                                     floatx4 (&z)[MB]) {
+  const auto [r, q] = lane_here();
 #pragma unroll
-  for (int rb = 0; rb < T / 16; ++rb)
+  for (int kb = 0; kb < NB; ++kb) {
+    floatx4 a[MB];
 #pragma unroll
-    for (int cb = 0; cb < CB; ++cb) {
-      floatx4 acc = {0.f, 0.f, 0.f, 0.f};
-      acc = mma_blk(sA + rb * 16 * lda, lda, 1, sW + cb * 16 * ldw, 1, ldw, K, acc);
-      if (kBias) {
-        const float b = bias[cb * 16 + r];
+    for (int mb = 0; mb < MB; ++mb)
+      a[mb] = *reinterpret_cast<const floatx4*>(sw + (16 * mb + r) * ld + 16 * kb + 4 * q);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) acc[e] += b;
-      }
-      z[rb][cb] = acc;
-    }
-}
-
-// y = G*W, G [T x K] in LDS (pitch ldg), W row-major [K][ldw]; CB output blocks.
-template <int T, int CB>
-__device__ __forceinline__ void gemm_gw(const float* sG, int ldg, const float* sW, int ldw,
-                                        int K, floatx4 (&y)[T / 16][CB]) {
+    for (int e = 0; e < 4; ++e)
 #pragma unroll
-  for (int rb = 0; rb < T / 16; ++rb)
-#pragma unroll
-    for (int cb = 0; cb < CB; ++cb) {
-      floatx4 acc = {0.f, 0.f, 0.f, 0.f};
-      y[rb][cb] = mma_blk(sG + rb * 16 * ldg, ldg, 1, sW + cb * 16, ldw, 1, K, acc);
-    }
-}
-
-// acc += G^T * A  (G [T x 16*OB] pitch ldg, A [T x 16*IB] pitch lda): weight gradient.
-template <int T, int OB, int IB>
-__device__ __forceinline__ void gemm_gtA(const float* sG, int ldg, const float* sA, int lda,
-                                         floatx4 (&acc)[OB][IB]) {
-#pragma unroll
-  for (int ob = 0; ob < OB; ++ob)
-#pragma unroll
-    for (int ib = 0; ib < IB; ++ib)
-      acc[ob][ib] = mma_blk(sG + ob * 16, 1, ldg, sA + ib * 16, lda, 1, T, acc[ob][ib]);
-}
-
-template <int T, int CB>
-__device__ __forceinline__ void store_frags(float* s, int ld, const floatx4 (&v)[T / 16][CB]) {
-  const int l = threadIdx.x & 63, r = l & 15, q = l >> 4;
-#pragma unroll
-  for (int rb = 0; rb < T / 16; ++rb)
-#pragma unroll
-    for (int cb = 0; cb < CB; ++cb)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) s[(rb * 16 + 4 * q + e) * ld + cb * 16 + r] = v[rb][cb][e];
-}
-
-// Column sums of fragments, added into per-lane partials (column cb*16 + r).
-template <int T, int CB>
-__device__ __forceinline__ void colsum_add(const floatx4 (&v)[T / 16][CB], float (&acc)[CB]) {
-#pragma unroll
-  for (int cb = 0; cb < CB; ++cb) {
-    float s = 0.f;
-#pragma unroll
-    for (int rb = 0; rb < T / 16; ++rb) s += v[rb][cb][0] + v[rb][cb][1] + v[rb][cb][2] + v[rb][cb][3];
-    acc[cb] += s;
+      for (int mb = 0; mb < MB; ++mb) z[mb] = mma(a[mb][e], b[kb][e], z[mb]);
+    __builtin_amdgcn_sched_barrier(0);
   }
 }
 
-// Writes one wavefront's gradient partial row in the packed layout.
-template <int H, int NH, int DP>
-__device__ void write_partial(float* __restrict__ out, int d, const floatx4 (&dW0)[H / 16][DP / 16],
-                              const floatx4 (&dW1)[H / 16][H / 16], const float (&db0)[H / 16],
-                              const float (&db1)[H / 16], const float (&dwo)[H / 16], float dbo) {
-  using M = Mlp<H, NH, DP>;
-  const int l = threadIdx.x & 63, r = l & 15, q = l >> 4;
+// z = W^T g (columns 16 c0 .. of W): NO blocks of 16 output dims.
+template <int NO, int MB>
+__device__ __forceinline__ void gemm_t(const float* __restrict__ sw, int ld, const float (&g)[MB][4],
+                                       floatx4 (&z)[NO]) {
+  const auto [r, q] = lane_here();
 #pragma unroll
-  for (int ob = 0; ob < M::HB; ++ob)
+  for (int i = 0; i < NO; ++i) z[i] = floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int ib = 0; ib < M::IB; ++ib)
+  for (int mo = 0; mo < MB; ++mo) {
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int o = ob * 16 + 4 * q + e, i = ib * 16 + r;
-        if (i < d) out[o * d + i] = dW0[ob][ib][e];
-      }
-  if (NH == 2) {
+    for (int e = 0; e < 4; ++e)
 #pragma unroll
-    for (int ob = 0; ob < M::HB; ++ob)
-#pragma unroll
-      for (int ib = 0; ib < M::HB; ++ib)
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          out[M::gW1(d) + (ob * 16 + 4 * q + e) * H + ib * 16 + r] = dW1[ob][ib][e];
+      for (int i = 0; i < NO; ++i)
+        z[i] = mma(sw[(16 * mo + 4 * q + e) * ld + 16 * i + r], g[mo][e], z[i]);
+    __builtin_amdgcn_sched_barrier(0);
   }
-#pragma unroll
-  for (int cb = 0; cb < M::HB; ++cb) {
-    const float s0 = sum4q(db0[cb]), s1 = sum4q(db1[cb]), so = sum4q(dwo[cb]);
-    if (q == 0) {
-      out[M::gB0(d) + cb * 16 + r] = s0;
-      if (NH == 2) out[M::gB1(d) + cb * 16 + r] = s1;
-      out[M::gWo(d) + cb * 16 + r] = so;
-    }
-  }
-  const float sbo = sum4q(dbo);
-  if (l == 0) out[M::gBo(d)] = sbo;
 }
 
-__device__ __forceinline__ int64_t count_of(const int32_t* n_dev, int64_t n_cap) {
-  if (!n_dev) return n_cap;
-  const int64_t v = *n_dev;
-  return v < 0 ? 0 : (v < n_cap ? v : n_cap);
+// Block starting values: a bias vector's rows (or zero).
+template <int MB>
+__device__ __forceinline__ void init_bias(const float* bias, floatx4 (&z)[MB]) {
+  const int q = lane_here().q;
+#pragma unroll
+  for (int mb = 0; mb < MB; ++mb) z[mb] = *reinterpret_cast<const floatx4*>(bias + 16 * mb + 4 * q);
+}
+template <int MB>
+__device__ __forceinline__ void init_zero(floatx4 (&z)[MB]) {
+#pragma unroll
+  for (int mb = 0; mb < MB; ++mb) z[mb] = floatx4{0.f, 0.f, 0.f, 0.f};
+}
+
+__device__ __forceinline__ float sum_q(float v) {  // over the 4 lanes of a point (same r)
+  v += __shfl_xor(v, 16, 64);
+  v += __shfl_xor(v, 32, 64);
+  return v;
+}
+__device__ __forceinline__ float sum_r(float v) {  // over the 16 points of a q group
+  v += __shfl_xor(v, 1, 64);
+  v += __shfl_xor(v, 2, 64);
+  v += __shfl_xor(v, 4, 64);
+  v += __shfl_xor(v, 8, 64);
+  return v;
 }
 
 // ----------------------------------------------------------------------------
-// Forward: sdf [n]; with dh0 != null also dsdf/dh0 [n, d] (backprop of 1).
+// Forward: sdf [n]; kGrad: also dsdf/dh0 [n, d] (backprop of 1).
 // ----------------------------------------------------------------------------
-template <int H, int NH, int DP, int T>
-__global__ void __launch_bounds__(64 * kWaves)
-mlp_fwd_kernel(const float* __restrict__ x, const float* __restrict__ enc, int E, int64_t n_cap,
-               const int32_t* __restrict__ n_dev, const float* __restrict__ mlp, float beta,
-               float* __restrict__ sdf_out, float* __restrict__ dh0) {
-  using M = Mlp<H, NH, DP>;
-  extern __shared__ float smem[];
-  float* sw = smem;
-  const int wid = threadIdx.x >> 6;
-  float* bufI = sw + M::kWFloats + wid * T * M::kRow;
-  float* bufA = bufI + T * M::LDI;
-  float* bufB = bufA + T * M::LDH;
+template <int H, int NH, int KB, bool kGrad>
+__global__ void __launch_bounds__(64 * kWaves, 4)
+mlp_fwd_kernel(const float* __restrict__ x, const float* __restrict__ enc, int E, int vec4,
+               int64_t n_cap, const int32_t* __restrict__ n_dev, const float* __restrict__ mlp,
+               float beta, float* __restrict__ sdf_out, float* __restrict__ dh0) {
+  using M = Mlp<H, NH, KB>;
+  constexpr int MB = M::MB;
+  extern __shared__ __attribute__((aligned(16))) float smem[];
+  load_weights<H, NH, KB>(smem, mlp, E);
+  const float* sW1 = smem + M::oW1;
+  const float* vec = smem + M::oVec;
+  const float inv_beta = 1.f / beta;
+  const int64_t n = dev_count(n_cap, n_dev);
+  const int l = threadIdx.x & 63, r = l & 15, q = l >> 4;
   const int d = 3 + E;
-  load_weights<H, NH, DP>(sw, mlp, d);
-  const int64_t n = count_of(n_dev, n_cap);
-  const int l = threadIdx.x & 63, r = l & 15, q = l >> 4;
-  const int64_t n_tiles = ceil_div(n, (int64_t)T * kWaves);
   __syncthreads();
-  for (int64_t tile = blockIdx.x; tile < n_tiles; tile += gridDim.x) {
-    const int64_t row0 = (tile * kWaves + wid) * T;
-    load_rows<DP, T>(bufI, x, enc, E, row0, n);
-    __syncthreads();
-    floatx4 z[T / 16][M::HB];
-    gemm_xwT<T, M::HB, true>(bufI, M::LDI, sw + M::oW0, M::LDI, sw + M::oB0, DP, z);
-    floatx4 z1[T / 16][M::HB];
+  const int64_t n_groups = ceil_div(n, 16), waves = (int64_t)gridDim.x * kWaves;
+  for (int64_t g = (int64_t)blockIdx.x * kWaves + (threadIdx.x >> 6); g < n_groups; g += waves) {
+    // weights re-read from LDS every group rather than held in registers
+    asm volatile("" ::: "memory");
+    const int64_t p = g * 16 + r;
+    const bool ok = p < n;
+    // the lane's quarter index and the encoding's shape, opaque in every step:
+    // the boundary tests of the loads and stores derive from them and are then
+    // evaluated where used instead of hoisted as dozens of execution masks
+    int qs = q, Es = E, v4s = vec4;
+    asm volatile("" : "+v"(qs), "+s"(Es), "+s"(v4s));
+    float h0[KB][4];
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb) load_in(x, enc, Es, v4s, p, ok, 16 * kb + 4 * qs, h0[kb]);
+    floatx4 z[MB];
+    init_bias<MB>(vec, z);
+    gemm<MB, KB>(smem, M::LD0, h0, z);
+    float d1[MB][4];
     if (NH == 2) {
+      float h1[MB][4];
 #pragma unroll
-      for (int rb = 0; rb < T / 16; ++rb)
-#pragma unroll
-        for (int cb = 0; cb < M::HB; ++cb) {
-          z1[rb][cb] = z[rb][cb];
-#pragma unroll
-          for (int e = 0; e < 4; ++e) z[rb][cb][e] = sp(z[rb][cb][e], beta);
-        }
-      store_frags<T, M::HB>(bufA, M::LDH, z);
-      __syncthreads();
-      gemm_xwT<T, M::HB, true>(bufA, M::LDH, sw + M::oW1, M::LDH, sw + M::oB1, H, z);
-    }
-    // output layer
-#pragma unroll
-    for (int rb = 0; rb < T / 16; ++rb)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        float p = 0.f;
-#pragma unroll
-        for (int cb = 0; cb < M::HB; ++cb) p += sp(z[rb][cb][e], beta) * sw[M::oWo + cb * 16 + r];
-        p = sum16(p) + sw[M::oBo];
-        const int64_t row = row0 + rb * 16 + 4 * q + e;
-        if (r == 0 && row < n) sdf_out[row] = p;
-      }
-    if (dh0) {
-      floatx4 g[T / 16][M::HB];
-#pragma unroll
-      for (int rb = 0; rb < T / 16; ++rb)
-#pragma unroll
-        for (int cb = 0; cb < M::HB; ++cb)
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-            g[rb][cb][e] = sw[M::oWo + cb * 16 + r] * sp_d(z[rb][cb][e], beta);
-      store_frags<T, M::HB>(bufB, M::LDH, g);
-      __syncthreads();
-      if (NH == 2) {
-        gemm_gw<T, M::HB>(bufB, M::LDH, sw + M::oW1, M::LDH, H, g);
-#pragma unroll
-        for (int rb = 0; rb < T / 16; ++rb)
-#pragma unroll
-          for (int cb = 0; cb < M::HB; ++cb)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) g[rb][cb][e] *= sp_d(z1[rb][cb][e], beta);
-        __syncthreads();
-        store_frags<T, M::HB>(bufB, M::LDH, g);
-        __syncthreads();
-      }
-      floatx4 gh0[T / 16][M::IB];
-      gemm_gw<T, M::IB>(bufB, M::LDH, sw + M::oW0, M::LDI, H, gh0);
-#pragma unroll
-      for (int rb = 0; rb < T / 16; ++rb)
-#pragma unroll
-        for (int ib = 0; ib < M::IB; ++ib)
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const int64_t row = row0 + rb * 16 + 4 * q + e;
-            const int c = ib * 16 + r;
-            if (row < n && c < d) dh0[row * d + c] = gh0[rb][ib][e];
-          }
-    }
-    __syncthreads();
-  }
-}
-
-// ----------------------------------------------------------------------------
-// Backward (sdf only): given dL/dsdf, the weight-gradient partials (one row
-// per wavefront) and dL/denc [n, E] (+ dL/dx [n,3] if requested).
-// ----------------------------------------------------------------------------
-template <int H, int NH, int DP, int T>
-__global__ void __launch_bounds__(64 * kWaves)
-mlp_bwd_kernel(const float* __restrict__ x, const float* __restrict__ enc, int E, int64_t n_cap,
-               const int32_t* __restrict__ n_dev, const float* __restrict__ mlp, float beta,
-               const float* __restrict__ g_sdf, float* __restrict__ g_enc,
-               float* __restrict__ g_x, float* __restrict__ partials) {
-  using M = Mlp<H, NH, DP>;
-  extern __shared__ float smem[];
-  float* sw = smem;
-  const int wid = threadIdx.x >> 6;
-  float* bufI = sw + M::kWFloats + wid * T * M::kRow;
-  float* bufA = bufI + T * M::LDI;
-  float* bufB = bufA + T * M::LDH;
-  const int d = 3 + E;
-  load_weights<H, NH, DP>(sw, mlp, d);
-  const int64_t n = count_of(n_dev, n_cap);
-  const int l = threadIdx.x & 63, r = l & 15, q = l >> 4;
-  const int64_t n_tiles = ceil_div(n, (int64_t)T * kWaves);
-  floatx4 dW0[M::HB][M::IB], dW1[M::HB][M::HB];
-#pragma unroll
-  for (int a = 0; a < M::HB; ++a) {
-#pragma unroll
-    for (int b = 0; b < M::IB; ++b) dW0[a][b] = floatx4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int b = 0; b < M::HB; ++b) dW1[a][b] = floatx4{0.f, 0.f, 0.f, 0.f};
-  }
-  float db0[M::HB], db1[M::HB], dwo[M::HB], dbo = 0.f;
-#pragma unroll
-  for (int a = 0; a < M::HB; ++a) db0[a] = db1[a] = dwo[a] = 0.f;
-  __syncthreads();
-  for (int64_t tile = blockIdx.x; tile < n_tiles; tile += gridDim.x) {
-    const int64_t row0 = (tile * kWaves + wid) * T;
-    load_rows<DP, T>(bufI, x, enc, E, row0, n);
-    __syncthreads();
-    floatx4 z[T / 16][M::HB], z1[T / 16][M::HB];
-    gemm_xwT<T, M::HB, true>(bufI, M::LDI, sw + M::oW0, M::LDI, sw + M::oB0, DP, z);
-    if (NH == 2) {
-      floatx4 h[T / 16][M::HB];
-#pragma unroll
-      for (int rb = 0; rb < T / 16; ++rb)
-#pragma unroll
-        for (int cb = 0; cb < M::HB; ++cb) {
-          z1[rb][cb] = z[rb][cb];
-#pragma unroll
-          for (int e = 0; e < 4; ++e) h[rb][cb][e] = sp(z[rb][cb][e], beta);
-        }
-      store_frags<T, M::HB>(bufA, M::LDH, h);
-      __syncthreads();
-      gemm_xwT<T, M::HB, true>(bufA, M::LDH, sw + M::oW1, M::LDH, sw + M::oB1, H, z);
-    }
-    // output layer: g_zL = gs * wo * s'(zL); dwo += gs * hL; dbo += gs
-    float gs[T / 16][4];
-#pragma unroll
-    for (int rb = 0; rb < T / 16; ++rb)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int64_t row = row0 + rb * 16 + 4 * q + e;
-        gs[rb][e] = row < n ? g_sdf[row] : 0.f;
-        dbo += (r == 0) ? gs[rb][e] : 0.f;
-      }
-    floatx4 g[T / 16][M::HB];
-#pragma unroll
-    for (int rb = 0; rb < T / 16; ++rb)
-#pragma unroll
-      for (int cb = 0; cb < M::HB; ++cb) {
-        const float w = sw[M::oWo + cb * 16 + r];
+      for (int mb = 0; mb < MB; ++mb) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          dwo[cb] += gs[rb][e] * sp(z[rb][cb][e], beta);
-          g[rb][cb][e] = gs[rb][e] * w * sp_d(z[rb][cb][e], beta);
+          const Sp s = softplus(z[mb][e], beta, inv_beta);
+          h1[mb][e] = s.h;
+          d1[mb][e] = s.d;
         }
+        __builtin_amdgcn_sched_barrier(0);
       }
-    store_frags<T, M::HB>(bufB, M::LDH, g);
-    __syncthreads();
-    if (NH == 2) {
-      colsum_add<T, M::HB>(g, db1);
-      gemm_gtA<T, M::HB, M::HB>(bufB, M::LDH, bufA, M::LDH, dW1);
-      gemm_gw<T, M::HB>(bufB, M::LDH, sw + M::oW1, M::LDH, H, g);
-#pragma unroll
-      for (int rb = 0; rb < T / 16; ++rb)
-#pragma unroll
-        for (int cb = 0; cb < M::HB; ++cb)
-#pragma unroll
-          for (int e = 0; e < 4; ++e) g[rb][cb][e] *= sp_d(z1[rb][cb][e], beta);
-      __syncthreads();
-      store_frags<T, M::HB>(bufB, M::LDH, g);
-      __syncthreads();
+      init_bias<MB>(vec + H, z);
+      gemm<MB, MB>(sW1, M::LD1, h1, z);
     }
-    colsum_add<T, M::HB>(g, db0);
-    gemm_gtA<T, M::HB, M::IB>(bufB, M::LDH, bufI, M::LDI, dW0);
-    if (g_enc || g_x) {
-      floatx4 gh0[T / 16][M::IB];
-      gemm_gw<T, M::IB>(bufB, M::LDH, sw + M::oW0, M::LDI, H, gh0);
+    float f = 0.f, gz[MB][4];
 #pragma unroll
-      for (int rb = 0; rb < T / 16; ++rb)
+    for (int mb = 0; mb < MB; ++mb) {
+      const floatx4 wo = *reinterpret_cast<const floatx4*>(vec + 2 * H + 16 * mb + 4 * q);
 #pragma unroll
-        for (int ib = 0; ib < M::IB; ++ib)
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const int64_t row = row0 + rb * 16 + 4 * q + e;
-            const int c = ib * 16 + r;
-            if (row < n) {
-              if (c < 3) {
-                if (g_x) g_x[row * 3 + c] = gh0[rb][ib][e];
-              } else if (c < d && g_enc) {
-                g_enc[row * E + (c - 3)] = gh0[rb][ib][e];
-              }
-            }
-          }
+      for (int e = 0; e < 4; ++e) {
+        const Sp s = softplus(z[mb][e], beta, inv_beta);
+        f += wo[e] * s.h;
+        gz[mb][e] = wo[e] * s.d;
+      }
+      __builtin_amdgcn_sched_barrier(0);
     }
-    __syncthreads();
+    f = sum_q(f) + vec[3 * H];
+    if (q == 0 && ok) sdf_out[p] = f;
+    if constexpr (kGrad) {
+      if (NH == 2) {
+        gemm_t<MB, MB>(sW1, M::LD1, gz, z);
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) gz[mb][e] = z[mb][e] * d1[mb][e];
+      }
+      floatx4 gi[KB];
+      gemm_t<KB, MB>(smem, M::LD0, gz, gi);
+#pragma unroll
+      for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int col = in_col(16 * kb + 4 * qs + e, Es);
+          if (ok && col >= 0) dh0[p * d + col] = gi[kb][e];
+        }
+    }
   }
-  // (dbo was counted once per row by the r == 0 lanes)
-  write_partial<H, NH, DP>(partials + (int64_t)(blockIdx.x * kWaves + wid) * M::n_params(d), d,
-                           dW0, dW1, db0, db1, dwo, dbo);
+}
+
+// ----------------------------------------------------------------------------
+// Weight-gradient helpers.  A workgroup steps over 64 points (16 per
+// wavefront): block tiles hold rows of 64 points (pitch 68 floats: a
+// wavefront's writes and its 16-byte operand reads are conflict-free).
+// ----------------------------------------------------------------------------
+template <int TP, int NB>
+__device__ __forceinline__ void tile_store(float* t, const float (&v)[NB][4]) {
+  const auto [r, q] = lane_here();
+  const int col = 16 * (threadIdx.x >> 6) + r;
+#pragma unroll
+  for (int b = 0; b < NB; ++b)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) t[(16 * b + 4 * q + e) * TP + col] = v[b][e];
+}
+
+// acc[t] += A[row block ia(t)] * B[row block ib(t)]^T over the step's points,
+// one of the two row blocks the same for every t.
+template <int TP, int T, bool kAFixed>
+__device__ __forceinline__ void tile_mma(const float* tA, const float* tB, int fixed, int first,
+                                         int stride, int n_blocks, floatx4 (&acc)[T]) {
+  const auto [r, q] = lane_here();
+  const float* tF = kAFixed ? tA : tB;
+  const float* tV = kAFixed ? tB : tA;
+#pragma unroll
+  for (int k = 0; k < kWaves; ++k) {
+    const floatx4 f = *reinterpret_cast<const floatx4*>(tF + (16 * fixed + r) * TP + 16 * k + 4 * q);
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+      const int b = first + stride * t;  // uniform
+      if (b >= n_blocks) continue;
+      const floatx4 v = *reinterpret_cast<const floatx4*>(tV + (16 * b + r) * TP + 16 * k + 4 * q);
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        acc[t] = kAFixed ? mma(f[e], v[e], acc[t]) : mma(v[e], f[e], acc[t]);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  }
+}
+
+// The workgroup's partial row of the weight gradient (packed layout): weight
+// blocks from the wavefronts that own them, vector sums combined over the
+// wavefronts in a fixed order through LDS (red: >= kWaves (3H + 1) floats no
+// longer in use).  Called by every lane of the workgroup.
+template <int H, int NH, int KB>
+__device__ __forceinline__ void write_partial(float* __restrict__ out, int E, int wid, float* red,
+                                              const floatx4 (&acc1)[Mlp<H, NH, KB>::T1],
+                                              const floatx4 (&acc0)[Mlp<H, NH, KB>::T0],
+                                              const float (&db0)[H / 16][4],
+                                              const float (&db1)[H / 16][4],
+                                              const float (&dwo)[H / 16][4], float dbo) {
+  using M = Mlp<H, NH, KB>;
+  constexpr int MB = M::MB;
+  const int l = threadIdx.x & 63, r = l & 15, q = l >> 4, d = 3 + E;
+#pragma unroll
+  for (int t = 0; t < M::T0; ++t) {
+    const int md = wid / MB + M::S * t, ob = wid % MB;
+    if (md >= KB) continue;
+    const int col = in_col(16 * md + r, E);
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (col >= 0) out[(16 * ob + 4 * q + e) * d + col] = acc0[t][e];
+  }
+  if (NH == 2) {
+#pragma unroll
+    for (int t = 0; t < M::T1; ++t) {
+      const int ob = wid / MB + M::S * t, ib = wid % MB;
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        out[M::gW1(d) + (16 * ob + 4 * q + e) * H + 16 * ib + r] = acc1[t][e];
+    }
+  }
+  float* mine = red + wid * (3 * H + 1);
+#pragma unroll
+  for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int u = 16 * mb + 4 * q + e;
+      const float s0 = sum_r(db0[mb][e]), s1 = sum_r(db1[mb][e]), so = sum_r(dwo[mb][e]);
+      if (r == 0) {
+        mine[u] = s0;
+        mine[H + u] = s1;
+        mine[2 * H + u] = so;
+      }
+    }
+  const float sbo = sum_q(sum_r(dbo));
+  if (l == 0) mine[3 * H] = sbo;
+  __syncthreads();
+  for (int t = threadIdx.x; t < 3 * H + 1; t += blockDim.x) {
+    float v = 0.f;
+    for (int w = 0; w < kWaves; ++w) v += red[w * (3 * H + 1) + t];
+    if (t < H) out[M::gB0(d) + t] = v;
+    else if (t < 2 * H) { if (NH == 2) out[M::gB1(d) + t - H] = v; }
+    else if (t < 3 * H) out[M::gWo(d) + t - 2 * H] = v;
+    else out[M::gBo(d)] = v;
+  }
+}
+
+// Stores 4 input dims c4..c4+3 of point p: encoding columns to g_enc, position
+// columns to g_x (either may be null).
+__device__ __forceinline__ void store_in(float* __restrict__ g_enc, float* __restrict__ g_x, int E,
+                                         int vec4, int64_t p, bool ok, int c4, floatx4 v) {
+  if (!ok) return;
+  if (vec4) {
+    if (c4 < E) {
+      if (g_enc) *reinterpret_cast<float4*>(g_enc + p * E + c4) = float4{v[0], v[1], v[2], v[3]};
+    } else if (c4 == E && g_x) {
+      g_x[p * 3] = v[0];
+      g_x[p * 3 + 1] = v[1];
+      g_x[p * 3 + 2] = v[2];
+    }
+    return;
+  }
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const int c = c4 + e;
+    if (c < E) {
+      if (g_enc) g_enc[p * E + c] = v[e];
+    } else if (c < E + 3 && g_x) {
+      g_x[p * 3 + (c - E)] = v[e];
+    }
+  }
+}
+
+// ----------------------------------------------------------------------------
+// Backward (sdf only): given dL/dsdf, one weight-gradient partial row per
+// workgroup and dL/denc [n, E] (+ dL/dx [n,3] if requested).
+// ----------------------------------------------------------------------------
+template <int H, int NH, int KB>
+__global__ void __launch_bounds__(64 * kWaves, 2)
+mlp_bwd_kernel(const float* __restrict__ x, const float* __restrict__ enc, int E, int vec4,
+               int64_t n_cap, const int32_t* __restrict__ n_dev, const float* __restrict__ mlp,
+               float beta, const float* __restrict__ g_sdf, float* __restrict__ g_enc,
+               float* __restrict__ g_x, float* __restrict__ partials) {
+  using M = Mlp<H, NH, KB>;
+  constexpr int MB = M::MB, TP = M::kTileP;
+  extern __shared__ __attribute__((aligned(16))) float smem[];
+  load_weights<H, NH, KB>(smem, mlp, E);
+  const float* sW1 = smem + M::oW1;
+  const float* vec = smem + M::oVec;
+  float* tA = smem + M::oTA;
+  float* tB = smem + M::oTB;
+  const float inv_beta = 1.f / beta;
+  const int64_t n = dev_count(n_cap, n_dev);
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int l = threadIdx.x & 63, r = l & 15, q = l >> 4;
+  const int fixed = wid % MB, first = wid / MB;
+  floatx4 acc1[M::T1], acc0[M::T0];
+  init_zero<M::T1>(acc1);
+  init_zero<M::T0>(acc0);
+  float db0[MB][4], db1[MB][4], dwo[MB][4], dbo = 0.f;
+#pragma unroll
+  for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) db0[mb][e] = db1[mb][e] = dwo[mb][e] = 0.f;
+  __syncthreads();
+  const int64_t n_steps = ceil_div(n, (int64_t)16 * kWaves);
+  for (int64_t step = blockIdx.x; step < n_steps; step += gridDim.x) {
+    const int64_t p = (step * kWaves + wid) * 16 + r;
+    const bool ok = p < n;
+    int qs = q, Es = E, v4s = vec4;  // opaque: see mlp_fwd_kernel
+    asm volatile("" : "+v"(qs), "+s"(Es), "+s"(v4s));
+    float h0[KB][4];
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb) load_in(x, enc, Es, v4s, p, ok, 16 * kb + 4 * qs, h0[kb]);
+    const float gs = ok ? g_sdf[p] : 0.f;
+    if (q == 0) dbo += gs;
+    floatx4 z[MB];
+    init_bias<MB>(vec, z);
+    gemm<MB, KB>(smem, M::LD0, h0, z);
+    float h1[MB][4], d1[MB][4], gz[MB][4];
+    if (NH == 2) {
+#pragma unroll
+      for (int mb = 0; mb < MB; ++mb) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const Sp s = softplus(z[mb][e], beta, inv_beta);
+          h1[mb][e] = s.h;
+          d1[mb][e] = s.d;
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      init_bias<MB>(vec + H, z);
+      gemm<MB, MB>(sW1, M::LD1, h1, z);
+    }
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) {
+      const floatx4 wo = *reinterpret_cast<const floatx4*>(vec + 2 * H + 16 * mb + 4 * q);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const Sp s = softplus(z[mb][e], beta, inv_beta);
+        dwo[mb][e] += gs * s.h;
+        gz[mb][e] = gs * wo[e] * s.d;
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if (NH == 2) {
+#pragma unroll
+      for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) db1[mb][e] += gz[mb][e];
+      tile_store<TP, MB>(tA, gz);
+      tile_store<TP, MB>(tB, h1);
+      __syncthreads();
+      tile_mma<TP, M::T1, false>(tA, tB, fixed, first, M::S, MB, acc1);
+      gemm_t<MB, MB>(sW1, M::LD1, gz, z);
+#pragma unroll
+      for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) gz[mb][e] = z[mb][e] * d1[mb][e];
+      __syncthreads();  // every wavefront is done reading the tiles
+    }
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) db0[mb][e] += gz[mb][e];
+    tile_store<TP, MB>(tA, gz);
+    tile_store<TP, KB>(tB, h0);
+    __syncthreads();
+    tile_mma<TP, M::T0, true>(tA, tB, fixed, first, M::S, KB, acc0);
+    if (g_enc || g_x) {
+      floatx4 gi[KB];
+      gemm_t<KB, MB>(smem, M::LD0, gz, gi);
+#pragma unroll
+      for (int kb = 0; kb < KB; ++kb)
+        store_in(g_enc, g_x, Es, v4s, p, ok, 16 * kb + 4 * qs, gi[kb]);
+    }
+    __syncthreads();  // tiles are rewritten by the next step
+  }
+  write_partial<H, NH, KB>(partials + (int64_t)blockIdx.x * M::n_params(3 + E), E, wid, tA, acc1,
+                           acc0, db0, db1, dwo, dbo);
 }
 
 // ----------------------------------------------------------------------------
 // Backward of J = sum_p a_p sdf(x_p) + v_p . grad_x sdf(x_p) (the analytic
 // gradient trained through its value, fields.py:107-119 with create_graph):
-// forward-over-reverse.  Tangents along v: hd0 = [v, encd] where encd is the
+// forward-over-reverse.  Tangents along v: hd0 = [encd, v] where encd is the
 // directional derivative of enc along v (from the hash-grid kernel).  Outputs
-// the weight-gradient partials, gb_h0 = dJ/dh0 and gt_h0 = dJ/dhd0 (both [n, d]).
+// the weight-gradient partials, gb_h0 = dJ/dh0 and gt_h0 = dJ/dhd0: rows of
+// out_ld floats in the packed column order, without the first out_c0 columns.
+// The weight gradient gb (x) h + gt (x) hd goes through the two tiles in turn,
+// so that two workgroups fit a CU.
 // ----------------------------------------------------------------------------
-template <int H, int NH, int DP, int T>
-__global__ void __launch_bounds__(64 * kWaves)
-mlp_bwd_ad_kernel(const float* __restrict__ x, const float* __restrict__ enc, const float* __restrict__ v,
-                  const float* __restrict__ encd, int E, int64_t n_cap,
-                  const int32_t* __restrict__ n_dev, const float* __restrict__ mlp, float beta,
-                  const float* __restrict__ a_sdf, float* __restrict__ gb_h0,
+template <int H, int NH, int KB>
+__global__ void __launch_bounds__(64 * kWaves, 2)
+mlp_bwd_ad_kernel(const float* __restrict__ x, const float* __restrict__ enc,
+                  const float* __restrict__ v, const float* __restrict__ encd, int E, int vec4,
+                  int64_t n_cap, const int32_t* __restrict__ n_dev, const float* __restrict__ mlp,
+                  float beta, const float* __restrict__ a_sdf, float* __restrict__ gb_h0,
                   float* __restrict__ gt_h0, float* __restrict__ partials, int out_ld,
                   int out_c0) {
-  using M = Mlp<H, NH, DP>;
-  extern __shared__ float smem[];
-  float* sw = smem;
-  const int wid = threadIdx.x >> 6;
-  float* bufI = sw + M::kWFloats + wid * 2 * T * M::kRow;
-  float* bufA = bufI + T * M::LDI;
-  float* bufB = bufA + T * M::LDH;
-  float* tbufI = bufB + T * M::LDH;
-  float* tbufA = tbufI + T * M::LDI;
-  float* tbufB = tbufA + T * M::LDH;
-  const int d = 3 + E;
-  load_weights<H, NH, DP>(sw, mlp, d);
-  const int64_t n = count_of(n_dev, n_cap);
+  using M = Mlp<H, NH, KB>;
+  constexpr int MB = M::MB, TP = M::kTileP;
+  extern __shared__ __attribute__((aligned(16))) float smem[];
+  load_weights<H, NH, KB>(smem, mlp, E);
+  const float* sW1 = smem + M::oW1;
+  const float* vec = smem + M::oVec;
+  float* tA = smem + M::oTA;
+  float* tB = smem + M::oTB;
+  const float inv_beta = 1.f / beta;
+  const int64_t n = dev_count(n_cap, n_dev);
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int l = threadIdx.x & 63, r = l & 15, q = l >> 4;
-  const int64_t n_tiles = ceil_div(n, (int64_t)T * kWaves);
-  floatx4 dW0[M::HB][M::IB], dW1[M::HB][M::HB];
+  const int fixed = wid % MB, first = wid / MB;
+  floatx4 acc1[M::T1], acc0[M::T0];
+  init_zero<M::T1>(acc1);
+  init_zero<M::T0>(acc0);
+  float db0[MB][4], db1[MB][4], dwo[MB][4], dbo = 0.f;
 #pragma unroll
-  for (int a = 0; a < M::HB; ++a) {
+  for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
-    for (int b = 0; b < M::IB; ++b) dW0[a][b] = floatx4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int b = 0; b < M::HB; ++b) dW1[a][b] = floatx4{0.f, 0.f, 0.f, 0.f};
-  }
-  float db0[M::HB], db1[M::HB], dwo[M::HB], dbo = 0.f;
-#pragma unroll
-  for (int a = 0; a < M::HB; ++a) db0[a] = db1[a] = dwo[a] = 0.f;
+    for (int e = 0; e < 4; ++e) db0[mb][e] = db1[mb][e] = dwo[mb][e] = 0.f;
   __syncthreads();
-  for (int64_t tile = blockIdx.x; tile < n_tiles; tile += gridDim.x) {
-    const int64_t row0 = (tile * kWaves + wid) * T;
-    load_rows<DP, T>(bufI, x, enc, E, row0, n);
-    load_rows<DP, T>(tbufI, v, encd, E, row0, n);
-    __syncthreads();
-    floatx4 z[T / 16][M::HB], zd[T / 16][M::HB], z1[T / 16][M::HB], z1d[T / 16][M::HB];
-    gemm_xwT<T, M::HB, true>(bufI, M::LDI, sw + M::oW0, M::LDI, sw + M::oB0, DP, z);
-    gemm_xwT<T, M::HB, false>(tbufI, M::LDI, sw + M::oW0, M::LDI, nullptr, DP, zd);
+  const int64_t n_steps = ceil_div(n, (int64_t)16 * kWaves);
+  for (int64_t step = blockIdx.x; step < n_steps; step += gridDim.x) {
+    const int64_t p = (step * kWaves + wid) * 16 + r;
+    const bool ok = p < n;
+    int qs = q, Es = E, v4s = vec4;  // opaque: see mlp_fwd_kernel
+    asm volatile("" : "+v"(qs), "+s"(Es), "+s"(v4s));
+    const float as = ok ? a_sdf[p] : 0.f;
+    if (q == 0) dbo += as;
+    floatx4 z[MB], zd[MB];
+    {
+      float h0[KB][4];
+#pragma unroll
+      for (int kb = 0; kb < KB; ++kb) load_in(x, enc, Es, v4s, p, ok, 16 * kb + 4 * qs, h0[kb]);
+      init_bias<MB>(vec, z);
+      gemm<MB, KB>(smem, M::LD0, h0, z);
+#pragma unroll
+      for (int kb = 0; kb < KB; ++kb) load_in(v, encd, Es, v4s, p, ok, 16 * kb + 4 * qs, h0[kb]);
+      init_zero<MB>(zd);
+      gemm<MB, KB>(smem, M::LD0, h0, zd);
+    }
+    // derivatives and tangent of layer 0 (NH == 2), cotangents of the value
+    // (gb) and of the tangent (gt) of the current layer's pre-activation
+    float d1[MB][4], w1[MB][4], gb[MB][4], gt[MB][4];  // w1 = zd0 s''(z0)
+    float h1[MB][4], hd1[MB][4];
     if (NH == 2) {
-      floatx4 h[T / 16][M::HB], hd[T / 16][M::HB];
 #pragma unroll
-      for (int rb = 0; rb < T / 16; ++rb)
+      for (int mb = 0; mb < MB; ++mb) {
 #pragma unroll
-        for (int cb = 0; cb < M::HB; ++cb) {
-          z1[rb][cb] = z[rb][cb];
-          z1d[rb][cb] = zd[rb][cb];
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            h[rb][cb][e] = sp(z[rb][cb][e], beta);
-            hd[rb][cb][e] = sp_d(z[rb][cb][e], beta) * zd[rb][cb][e];
-          }
+        for (int e = 0; e < 4; ++e) {
+          const Sp s = softplus<true>(z[mb][e], beta, inv_beta);
+          h1[mb][e] = s.h;
+          d1[mb][e] = s.d;
+          w1[mb][e] = zd[mb][e] * (beta * s.d * s.c);
+          hd1[mb][e] = s.d * zd[mb][e];
         }
-      store_frags<T, M::HB>(bufA, M::LDH, h);
-      store_frags<T, M::HB>(tbufA, M::LDH, hd);
-      __syncthreads();
-      gemm_xwT<T, M::HB, true>(bufA, M::LDH, sw + M::oW1, M::LDH, sw + M::oB1, H, z);
-      gemm_xwT<T, M::HB, false>(tbufA, M::LDH, sw + M::oW1, M::LDH, nullptr, H, zd);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      init_bias<MB>(vec + H, z);
+      gemm<MB, MB>(sW1, M::LD1, h1, z);
+      init_zero<MB>(zd);
+      gemm<MB, MB>(sW1, M::LD1, hd1, zd);
+      tile_store<TP, MB>(tB, h1);
     }
     // output: J = a*(wo.hL + bo) + wo.hdL;  gb_zL = a wo s' + wo zdL s'';  gt_zL = wo s'
-    float as[T / 16][4];
 #pragma unroll
-    for (int rb = 0; rb < T / 16; ++rb)
+    for (int mb = 0; mb < MB; ++mb) {
+      const floatx4 wo = *reinterpret_cast<const floatx4*>(vec + 2 * H + 16 * mb + 4 * q);
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const int64_t row = row0 + rb * 16 + 4 * q + e;
-        as[rb][e] = row < n ? a_sdf[row] : 0.f;
-        dbo += (r == 0) ? as[rb][e] : 0.f;
+        const Sp s = softplus<true>(z[mb][e], beta, inv_beta);
+        dwo[mb][e] += as * s.h + s.d * zd[mb][e];
+        gb[mb][e] = as * wo[e] * s.d + wo[e] * zd[mb][e] * (beta * s.d * s.c);
+        gt[mb][e] = wo[e] * s.d;
       }
-    floatx4 gb[T / 16][M::HB], gt[T / 16][M::HB];
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if (NH == 2) {
 #pragma unroll
-    for (int rb = 0; rb < T / 16; ++rb)
+      for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
-      for (int cb = 0; cb < M::HB; ++cb) {
-        const float w = sw[M::oWo + cb * 16 + r];
+        for (int e = 0; e < 4; ++e) db1[mb][e] += gb[mb][e];
+      tile_store<TP, MB>(tA, gb);
+      __syncthreads();
+      tile_mma<TP, M::T1, false>(tA, tB, fixed, first, M::S, MB, acc1);
+      __syncthreads();  // every wavefront is done reading the tiles
+      tile_store<TP, MB>(tA, gt);
+      tile_store<TP, MB>(tB, hd1);
+      gemm_t<MB, MB>(sW1, M::LD1, gb, z);
+      gemm_t<MB, MB>(sW1, M::LD1, gt, zd);
+      __syncthreads();
+      tile_mma<TP, M::T1, false>(tA, tB, fixed, first, M::S, MB, acc1);
+#pragma unroll
+      for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          const float zz = z[rb][cb][e], s1 = sp_d(zz, beta);
-          dwo[cb] += as[rb][e] * sp(zz, beta) + s1 * zd[rb][cb][e];
-          gb[rb][cb][e] = as[rb][e] * w * s1 + w * zd[rb][cb][e] * sp_dd(zz, beta);
-          gt[rb][cb][e] = w * s1;
+          gb[mb][e] = z[mb][e] * d1[mb][e] + zd[mb][e] * w1[mb][e];
+          gt[mb][e] = zd[mb][e] * d1[mb][e];
         }
-      }
-    store_frags<T, M::HB>(bufB, M::LDH, gb);
-    store_frags<T, M::HB>(tbufB, M::LDH, gt);
-    __syncthreads();
-    if (NH == 2) {
-      colsum_add<T, M::HB>(gb, db1);
-      gemm_gtA<T, M::HB, M::HB>(bufB, M::LDH, bufA, M::LDH, dW1);
-      gemm_gtA<T, M::HB, M::HB>(tbufB, M::LDH, tbufA, M::LDH, dW1);
-      gemm_gw<T, M::HB>(bufB, M::LDH, sw + M::oW1, M::LDH, H, gb);
-      gemm_gw<T, M::HB>(tbufB, M::LDH, sw + M::oW1, M::LDH, H, gt);
-#pragma unroll
-      for (int rb = 0; rb < T / 16; ++rb)
-#pragma unroll
-        for (int cb = 0; cb < M::HB; ++cb)
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const float zz = z1[rb][cb][e], s1 = sp_d(zz, beta);
-            gb[rb][cb][e] = gb[rb][cb][e] * s1 + gt[rb][cb][e] * z1d[rb][cb][e] * sp_dd(zz, beta);
-            gt[rb][cb][e] = gt[rb][cb][e] * s1;
-          }
-      __syncthreads();
-      store_frags<T, M::HB>(bufB, M::LDH, gb);
-      store_frags<T, M::HB>(tbufB, M::LDH, gt);
       __syncthreads();
     }
-    colsum_add<T, M::HB>(gb, db0);
-    gemm_gtA<T, M::HB, M::IB>(bufB, M::LDH, bufI, M::LDI, dW0);
-    gemm_gtA<T, M::HB, M::IB>(tbufB, M::LDH, tbufI, M::LDI, dW0);
-    floatx4 o1[T / 16][M::IB], o2[T / 16][M::IB];
-    gemm_gw<T, M::IB>(bufB, M::LDH, sw + M::oW0, M::LDI, H, o1);
-    gemm_gw<T, M::IB>(tbufB, M::LDH, sw + M::oW0, M::LDI, H, o2);
 #pragma unroll
-    for (int rb = 0; rb < T / 16; ++rb)
+    for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
-      for (int ib = 0; ib < M::IB; ++ib)
+      for (int e = 0; e < 4; ++e) db0[mb][e] += gb[mb][e];
+    // layer 0's weights: gb (x) h0, then gt (x) hd0 (the inputs read again)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int64_t row = row0 + rb * 16 + 4 * q + e;
-          const int c = ib * 16 + r;
-          if (row < n && c < d && c >= out_c0) {
-            if (gb_h0) gb_h0[row * out_ld + (c - out_c0)] = o1[rb][ib][e];
-            if (gt_h0) gt_h0[row * out_ld + (c - out_c0)] = o2[rb][ib][e];
-          }
+    for (int pass = 0; pass < 2; ++pass) {
+      float h0[KB][4];
+#pragma unroll
+      for (int kb = 0; kb < KB; ++kb)
+        load_in(pass ? v : x, pass ? encd : enc, Es, v4s, p, ok, 16 * kb + 4 * qs, h0[kb]);
+      tile_store<TP, MB>(tA, pass ? gt : gb);
+      tile_store<TP, KB>(tB, h0);
+      __syncthreads();
+      tile_mma<TP, M::T0, true>(tA, tB, fixed, first, M::S, KB, acc0);
+      float* out = pass ? gt_h0 : gb_h0;
+      if (out) {
+        floatx4 gi[KB];
+        gemm_t<KB, MB>(smem, M::LD0, pass ? gt : gb, gi);
+        if (out_c0 == 3) {
+          // the encoding's columns alone
+#pragma unroll
+          for (int kb = 0; kb < KB; ++kb)
+            store_in(out, nullptr, Es, v4s, p, ok, 16 * kb + 4 * qs, gi[kb]);
+        } else {
+#pragma unroll
+          for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              const int col = in_col(16 * kb + 4 * qs + e, Es);
+              if (ok && col >= 0) out[p * out_ld + col] = gi[kb][e];
+            }
         }
-    __syncthreads();
+      }
+      __syncthreads();  // tiles are rewritten by the next pass
+    }
   }
-  write_partial<H, NH, DP>(partials + (int64_t)(blockIdx.x * kWaves + wid) * M::n_params(d), d,
-                           dW0, dW1, db0, db1, dwo, dbo);
+  write_partial<H, NH, KB>(partials + (int64_t)blockIdx.x * M::n_params(3 + E), E, wid, tA, acc1,
+                           acc0, db0, db1, dwo, dbo);
 }
 
 // Column sums of the partial rows in a fixed order: a workgroup owns 64
@@ -641,10 +757,12 @@ int mlp_reduce_rows(const float* part, int64_t rows, int cols, float* out, int a
 // ---------------------------------------------------------------------------
 // dispatch
 // ---------------------------------------------------------------------------
-constexpr int kGridMax = 256;
+// workgroups: 4 of the forward and 2 of the backward fit a CU (LDS)
+constexpr int kFwdBlocksMax = 256 * 4;
+constexpr int kBwdBlocksMax = 256 * 2;
 
 struct MlpCfg {
-  int H, NH, DP, d;
+  int H, NH, KB, d;
 };
 
 static int mlp_cfg(const char* who, int E, int H, int NH, MlpCfg* c) {
@@ -654,29 +772,24 @@ static int mlp_cfg(const char* who, int E, int H, int NH, MlpCfg* c) {
   c->H = H;
   c->NH = NH;
   c->d = 3 + E;
-  c->DP = c->d <= 32 ? 32 : (c->d <= 48 ? 48 : 64);
+  c->KB = c->d <= 32 ? 2 : (c->d <= 48 ? 3 : 4);
   return SN_OK;
-}
-
-template <int H, int NH, int DP>
-constexpr size_t smem_bytes(int T, int nbuf) {
-  return sizeof(float) * (Mlp<H, NH, DP>::kWFloats + (size_t)kWaves * nbuf * T * Mlp<H, NH, DP>::kRow);
 }
 
 #define SN_MLP_DISPATCH(c, ...)                                                        \
   do {                                                                                 \
-    if (c.H == 32 && c.NH == 1 && c.DP == 32) { constexpr int kH = 32, kNH = 1, kDP = 32; __VA_ARGS__; } \
-    else if (c.H == 32 && c.NH == 1 && c.DP == 48) { constexpr int kH = 32, kNH = 1, kDP = 48; __VA_ARGS__; } \
-    else if (c.H == 32 && c.NH == 1 && c.DP == 64) { constexpr int kH = 32, kNH = 1, kDP = 64; __VA_ARGS__; } \
-    else if (c.H == 32 && c.NH == 2 && c.DP == 32) { constexpr int kH = 32, kNH = 2, kDP = 32; __VA_ARGS__; } \
-    else if (c.H == 32 && c.NH == 2 && c.DP == 48) { constexpr int kH = 32, kNH = 2, kDP = 48; __VA_ARGS__; } \
-    else if (c.H == 32 && c.NH == 2 && c.DP == 64) { constexpr int kH = 32, kNH = 2, kDP = 64; __VA_ARGS__; } \
-    else if (c.H == 64 && c.NH == 1 && c.DP == 32) { constexpr int kH = 64, kNH = 1, kDP = 32; __VA_ARGS__; } \
-    else if (c.H == 64 && c.NH == 1 && c.DP == 48) { constexpr int kH = 64, kNH = 1, kDP = 48; __VA_ARGS__; } \
-    else if (c.H == 64 && c.NH == 1 && c.DP == 64) { constexpr int kH = 64, kNH = 1, kDP = 64; __VA_ARGS__; } \
-    else if (c.H == 64 && c.NH == 2 && c.DP == 32) { constexpr int kH = 64, kNH = 2, kDP = 32; __VA_ARGS__; } \
-    else if (c.H == 64 && c.NH == 2 && c.DP == 48) { constexpr int kH = 64, kNH = 2, kDP = 48; __VA_ARGS__; } \
-    else { constexpr int kH = 64, kNH = 2, kDP = 64; __VA_ARGS__; }                     \
+    if (c.H == 32 && c.NH == 1 && c.KB == 2) { constexpr int kH = 32, kNH = 1, kKB = 2; __VA_ARGS__; } \
+    else if (c.H == 32 && c.NH == 1 && c.KB == 3) { constexpr int kH = 32, kNH = 1, kKB = 3; __VA_ARGS__; } \
+    else if (c.H == 32 && c.NH == 1) { constexpr int kH = 32, kNH = 1, kKB = 4; __VA_ARGS__; } \
+    else if (c.H == 32 && c.KB == 2) { constexpr int kH = 32, kNH = 2, kKB = 2; __VA_ARGS__; } \
+    else if (c.H == 32 && c.KB == 3) { constexpr int kH = 32, kNH = 2, kKB = 3; __VA_ARGS__; } \
+    else if (c.H == 32) { constexpr int kH = 32, kNH = 2, kKB = 4; __VA_ARGS__; }      \
+    else if (c.NH == 1 && c.KB == 2) { constexpr int kH = 64, kNH = 1, kKB = 2; __VA_ARGS__; } \
+    else if (c.NH == 1 && c.KB == 3) { constexpr int kH = 64, kNH = 1, kKB = 3; __VA_ARGS__; } \
+    else if (c.NH == 1) { constexpr int kH = 64, kNH = 1, kKB = 4; __VA_ARGS__; }      \
+    else if (c.KB == 2) { constexpr int kH = 64, kNH = 2, kKB = 2; __VA_ARGS__; }      \
+    else if (c.KB == 3) { constexpr int kH = 64, kNH = 2, kKB = 3; __VA_ARGS__; }      \
+    else { constexpr int kH = 64, kNH = 2, kKB = 4; __VA_ARGS__; }                     \
   } while (0)
 
 // Blocks use more than the default 64 KB of dynamic LDS (gfx950 has 160 KB).
@@ -697,9 +810,14 @@ static void allow_smem(Kern k, size_t bytes) {
   }
 }
 
-static unsigned grid_blocks(int64_t n_cap, int T) {
-  int64_t b = ceil_div(n_cap > 0 ? n_cap : 1, (int64_t)T * kWaves);
-  return (unsigned)(b < kGridMax ? b : kGridMax);
+static unsigned grid_blocks(int64_t n_cap, int max_blocks) {
+  const int64_t b = ceil_div(n_cap > 0 ? n_cap : 1, (int64_t)16 * kWaves);
+  return (unsigned)(b < max_blocks ? b : max_blocks);
+}
+
+// float4 access to rows of E floats
+static int vec4_ok(const float* p, int E) {
+  return (E % 4 == 0) && ((uintptr_t)p % 16 == 0) ? 1 : 0;
 }
 
 }  // namespace sn
@@ -718,8 +836,8 @@ size_t sn_mlp_bwd_workspace_bytes(int64_t n_cap, int32_t enc_dims, int32_t d_hid
                                   int32_t n_layers, int32_t analytic) {
   int np = sn_mlp_n_params(3 + enc_dims, d_hidden, n_layers);
   if (np < 0) return 0;
-  const int T = analytic ? 16 : 32;
-  return (size_t)grid_blocks(n_cap, T) * kWaves * np * sizeof(float);
+  (void)analytic;
+  return (size_t)grid_blocks(n_cap, kBwdBlocksMax) * np * sizeof(float);
 }
 
 int sn_mlp_fwd(const float* x, const float* enc, int32_t enc_dims, int64_t n_cap,
@@ -732,13 +850,17 @@ int sn_mlp_fwd(const float* x, const float* enc, int32_t enc_dims, int64_t n_cap
   SN_REQUIRE(n_cap >= 0, "sn_mlp_fwd: n < 0");
   if (n_cap == 0) return SN_OK;
   SN_REQUIRE(x && mlp && sdf && (enc || enc_dims == 0), "sn_mlp_fwd: null pointer");
-  constexpr int T = 32;
   hipStream_t s = as_stream(stream);
+  const unsigned grid = grid_blocks(n_cap, kFwdBlocksMax);
+  const int v4 = vec4_ok(enc, enc_dims);
   SN_MLP_DISPATCH(c, {
-    const size_t sm = smem_bytes<kH, kNH, kDP>(T, 1);
-    allow_smem(mlp_fwd_kernel<kH, kNH, kDP, T>, sm);
-    mlp_fwd_kernel<kH, kNH, kDP, T><<<grid_blocks(n_cap, T), 64 * kWaves, sm, s>>>(
-        x, enc, enc_dims, n_cap, n_dev, mlp, beta, sdf, dsdf_dh0);
+    constexpr size_t sm = sizeof(float) * Mlp<kH, kNH, kKB>::kFwd;
+    if (dsdf_dh0)
+      mlp_fwd_kernel<kH, kNH, kKB, true><<<grid, 64 * kWaves, sm, s>>>(
+          x, enc, enc_dims, v4, n_cap, n_dev, mlp, beta, sdf, dsdf_dh0);
+    else
+      mlp_fwd_kernel<kH, kNH, kKB, false><<<grid, 64 * kWaves, sm, s>>>(
+          x, enc, enc_dims, v4, n_cap, n_dev, mlp, beta, sdf, nullptr);
   });
   return check_launch("sn_mlp_fwd");
 }
@@ -758,18 +880,18 @@ int sn_mlp_bwd(const float* x, const float* enc, int32_t enc_dims, int64_t n_cap
     set_error("sn_mlp_bwd: workspace %zu < %zu bytes", workspace_bytes, need);
     return SN_ESPACE;
   }
-  constexpr int T = 32;
   hipStream_t s = as_stream(stream);
   const int np = sn_mlp_n_params(c.d, d_hidden, n_layers);
-  const unsigned grid = grid_blocks(n_cap, T);
+  const unsigned grid = grid_blocks(n_cap, kBwdBlocksMax);
   float* part = reinterpret_cast<float*>(workspace);
+  const int v4 = vec4_ok(enc, enc_dims) && vec4_ok(g_enc, enc_dims);
   SN_MLP_DISPATCH(c, {
-    const size_t sm = smem_bytes<kH, kNH, kDP>(T, 1);
-    allow_smem(mlp_bwd_kernel<kH, kNH, kDP, T>, sm);
-    mlp_bwd_kernel<kH, kNH, kDP, T><<<grid, 64 * kWaves, sm, s>>>(
-        x, enc, enc_dims, n_cap, n_dev, mlp, beta, g_sdf, g_enc, g_x, part);
+    constexpr size_t sm = sizeof(float) * Mlp<kH, kNH, kKB>::kBwd;
+    allow_smem(mlp_bwd_kernel<kH, kNH, kKB>, sm);
+    mlp_bwd_kernel<kH, kNH, kKB><<<grid, 64 * kWaves, sm, s>>>(
+        x, enc, enc_dims, v4, n_cap, n_dev, mlp, beta, g_sdf, g_enc, g_x, part);
   });
-  if ((rc = mlp_reduce_rows(part, (int64_t)grid * kWaves, np, g_mlp, accumulate, s))) return rc;
+  if ((rc = mlp_reduce_rows(part, (int64_t)grid, np, g_mlp, accumulate, s))) return rc;
   return check_launch("sn_mlp_bwd");
 }
 
@@ -789,19 +911,20 @@ static int mlp_bwd_ad(const float* x, const float* enc, const float* v, const fl
     set_error("sn_mlp_bwd_ad: workspace %zu < %zu bytes", workspace_bytes, need);
     return SN_ESPACE;
   }
-  constexpr int T = 16;
   hipStream_t s = as_stream(stream);
   const int np = sn_mlp_n_params(c.d, d_hidden, n_layers);
-  const unsigned grid = grid_blocks(n_cap, T);
+  const unsigned grid = grid_blocks(n_cap, kBwdBlocksMax);
   float* part = reinterpret_cast<float*>(workspace);
+  const int v4 = vec4_ok(enc, enc_dims) && vec4_ok(enc_dot, enc_dims) &&
+                 (out_c0 != 3 || (vec4_ok(g_h0, enc_dims) && vec4_ok(g_h0_dot, enc_dims)));
   SN_MLP_DISPATCH(c, {
-    const size_t sm = smem_bytes<kH, kNH, kDP>(T, 2);
-    allow_smem(mlp_bwd_ad_kernel<kH, kNH, kDP, T>, sm);
-    mlp_bwd_ad_kernel<kH, kNH, kDP, T><<<grid, 64 * kWaves, sm, s>>>(
-        x, enc, v, enc_dot, enc_dims, n_cap, n_dev, mlp, beta, g_sdf, g_h0, g_h0_dot, part,
+    constexpr size_t sm = sizeof(float) * Mlp<kH, kNH, kKB>::kBwd;
+    allow_smem(mlp_bwd_ad_kernel<kH, kNH, kKB>, sm);
+    mlp_bwd_ad_kernel<kH, kNH, kKB><<<grid, 64 * kWaves, sm, s>>>(
+        x, enc, v, enc_dot, enc_dims, v4, n_cap, n_dev, mlp, beta, g_sdf, g_h0, g_h0_dot, part,
         out_ld, out_c0);
   });
-  if ((rc = mlp_reduce_rows(part, (int64_t)grid * kWaves, np, g_mlp, accumulate, s))) return rc;
+  if ((rc = mlp_reduce_rows(part, (int64_t)grid, np, g_mlp, accumulate, s))) return rc;
   return check_launch("sn_mlp_bwd_ad");
 }
 
