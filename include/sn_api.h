@@ -367,6 +367,19 @@ int sn_render_step(int32_t n_patches, int32_t patch_h, int32_t patch_w, const fl
                    float* g_sdf_starts, float* g_sdf_ends, float* g_grad_starts,
                    float* losses, float* partials, float* weight_sum, float* comp_normal,
                    void* stream);
+/* The same for SDF values of fp32 accuracy: opacities and mask loss without  */
+/* cancelling differences (their rounding is most of the gradients' error     */
+/* then, and lost in the SDF's own with fp16 weights).                        */
+int sn_render_step_fine(int32_t n_patches, int32_t patch_h, int32_t patch_w, const float* rays_o,
+                        const float* rays_d, const float* plane_n, const float* v_inv,
+                        const float* n_true, const float* mask, const int32_t* packed_info,
+                        const float* t_starts, const float* t_ends, const int32_t* diff_idx,
+                        const float* sdf_starts, const float* sdf_ends, const float* grad_starts,
+                        const float* inv_s, const float* mask_sum, const int32_t* n_samples,
+                        float normal_w, float eik_w, float mask_w, int32_t loss_l1,
+                        float* g_sdf_starts, float* g_sdf_ends, float* g_grad_starts,
+                        float* losses, float* partials, float* weight_sum, float* comp_normal,
+                        void* stream);
 
 /* The same MLP on the fp16 (forward) / bf16 (backward) matrix cores with  */
 /* fp32 accumulation: weights rounded once to the MFMA type, activations    */

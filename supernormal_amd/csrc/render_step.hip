@@ -29,6 +29,8 @@
 // divisions and square roots are the hardware reciprocal and square root (a few
 // ulp), not the correctly rounded sequences, which were a third of the sample-
 // parallel kernel's VALU instructions.
+#include <type_traits>
+
 #include "sn_common.h"
 
 namespace sn {
@@ -62,13 +64,110 @@ struct RenderArgs {
   float* comp_normal;      // [B, P, 3] (nullable)
 };
 
-__device__ __forceinline__ float sigmoidf_(float x) { return 1.f / (1.f + expf(-x)); }
+// Two forms of the opacity and of the mask loss, for SDF values of fp16 and of
+// fp32 accuracy (kFine).  The plain form's cancellations (1 - sum of weights of
+// an opaque ray, c - e and 1 - c outside the surface, dL/dw - Q) amplify the
+// rounding of the SDF and of the rendering itself to 1e-4 of the gradients,
+// 1e-3 of a grazing sample's: below what fp16 weights leave (2e-2), most of
+// the error with fp32 ones (1.8e-4 of an iteration's gradients against 64 bits,
+// 1e-5 with the fine form, whose terms cost the kernel 3 %).  The fine form has
+// no such difference: complements come from one exponential, 1 - sum of weights
+// is the transmittance behind the last sample (the weights telescope), and the
+// weight sum's part of dL/dalpha is g_ws T_end / (1 - alpha), outside the
+// recurrence (where g_ws is not 0, T_end >= 1e-5 and no alpha is 1).
+
+// Mask loss of a ray (binary cross entropy of the clipped weight sum,
+// exp_runner.py:193-196) and its gradient; T: transmittance behind the samples.
+struct MaskLoss {
+  float l, g;
+};
+template <bool kFine>
+__device__ __forceinline__ MaskLoss mask_loss(float ws, float T, float m, float mask_w,
+                                              float n_mask) {
+  const float lo = 1e-5f, hi = 1.f - 1e-5f;
+  const float xw = fminf(fmaxf(ws, lo), hi);
+  MaskLoss r;
+  if constexpr (kFine) {
+    const bool pass = ws >= lo && T >= lo;
+    const float om = ws < lo ? hi : fmaxf(T, lo);  // 1 - xw
+    r.l = -(m * fmaxf(logf(xw), -100.f) + (1.f - m) * fmaxf(logf(om), -100.f)) / n_mask;
+    // (xw - m) / (om xw) with m in {0, 1} or between
+    r.g = pass ? mask_w * ((1.f - m) * xw - m * om) / fmaxf(om * xw, 1e-12f) / n_mask : 0.f;
+  } else {
+    r.l = -(m * fmaxf(logf(xw), -100.f) + (1.f - m) * fmaxf(logf(1.f - xw), -100.f)) / n_mask;
+    const bool pass = ws >= lo && ws <= hi;
+    r.g = pass ? mask_w * (xw - m) / fmaxf((1.f - xw) * xw, 1e-12f) / n_mask : 0.f;
+  }
+  return r;
+}
+
+// Opacity of a sample from the SDF at its start and end (renderer.py:164-179):
+// c = sigma(s fs), e = sigma(s fe), r = (c - e + 1e-5) / (c + 1e-5), alpha =
+// clip(r, 0, 1), om = 1 - alpha; a lane without a sample (act false) is fully
+// transparent.  grad: dL/dfs, dL/dfe and the sample's part of dL/dinv_s from
+// dL/dalpha.
+template <bool kFine>
+struct Opacity;
+
+template <>
+struct Opacity<false> {
+  float alpha, om, c, e, r;
+  __device__ __forceinline__ Opacity(float fs, float fe, float inv_s, bool act) {
+    c = 1.f / (1.f + expf(-(fs * inv_s)));
+    e = 1.f / (1.f + expf(-(fe * inv_s)));
+    r = ((c - e) + 1e-5f) / (c + 1e-5f);
+    alpha = act ? fminf(fmaxf(r, 0.f), 1.f) : 0.f;
+    om = 1.f - alpha;
+  }
+  __device__ __forceinline__ void grad(float g_alpha, float fs, float fe, float inv_s, float& g_fs,
+                                       float& g_fe, float& g_inv) const {
+    const float gr = (r >= 0.f && r <= 1.f) ? g_alpha : 0.f;
+    const float den = c + 1e-5f;
+    const float g_c = gr * e / (den * den), g_e = -gr / den;
+    g_fs = g_c * inv_s * c * (1.f - c);
+    g_fe = g_e * inv_s * e * (1.f - e);
+    g_inv = g_c * fs * c * (1.f - c) + g_e * fe * e * (1.f - e);
+  }
+};
+
+// c1 = 1 - c, e1 = 1 - e from the same exponential; om = e / (c + 1e-5) where r
+// is not clipped; ac, ae: d alpha / d (s fs) and d alpha / d (s fe), zero where
+// it is.
+template <>
+struct Opacity<true> {
+  float alpha, om, ac, ae;
+  static __device__ __forceinline__ void sigmoid2(float x, float& c, float& c1) {
+    const float t = expf(-fabsf(x)), r = 1.f / (1.f + t), tr = t * r;
+    c = x > 0.f ? r : tr;
+    c1 = x > 0.f ? tr : r;
+  }
+  __device__ __forceinline__ Opacity(float fs, float fe, float inv_s, bool act) {
+    float c, c1, e, e1;
+    sigmoid2(fs * inv_s, c, c1);
+    sigmoid2(fe * inv_s, e, e1);
+    const float inv_den = 1.f / (c + 1e-5f), ed = e * inv_den;
+    const float r = ((fs > 0.f ? e1 - c1 : c - e) + 1e-5f) * inv_den;
+    const bool in = r >= 0.f && r <= 1.f;
+    alpha = act ? fminf(fmaxf(r, 0.f), 1.f) : 0.f;
+    om = act && r > 0.f && r < 1.f ? ed : 1.f - alpha;
+    ac = in ? ed * inv_den * (c * c1) : 0.f;
+    ae = in ? -inv_den * (e * e1) : 0.f;
+  }
+  __device__ __forceinline__ void grad(float g_alpha, float fs, float fe, float inv_s, float& g_fs,
+                                       float& g_fe, float& g_inv) const {
+    const float g_c = g_alpha * ac, g_e = g_alpha * ae;
+    g_fs = g_c * inv_s;
+    g_fe = g_e * inv_s;
+    g_inv = g_c * fs + g_e * fe;
+  }
+};
 
 // per (sample, ray) quantities of the forward model
 struct SampleF {
-  float fs, fe, ts, te, c, e, r, alpha, g[3], proj[3], dtd, denx, deny;
+  float fs, fe, ts, te, g[3], proj[3], dtd, denx, deny;
 };
 
+template <bool kFine>
 __global__ void __launch_bounds__(64)
 render_step_kernel(RenderArgs a) {
   const int lane = threadIdx.x & 63;
@@ -101,7 +200,8 @@ render_step_kernel(RenderArgs a) {
       d[c] = a.rays_d[(p * P + k) * 3 + c];
       nt[c] = a.n_true[(p * P + k) * 3 + c];
     }
-    for (int c = 0; c < 9; ++c) vi[c] = a.vinv[(p * P + k) * 9 + c];
+    if (!ad)  // ('ad' callers may leave it out)
+      for (int c = 0; c < 9; ++c) vi[c] = a.vinv[(p * P + k) * 9 + c];
     m = a.mask[p * P + k];
     const float* n = a.plane_n + 3 * p;
     const float* dc = a.rays_d + (p * P + kc) * 3;
@@ -135,10 +235,6 @@ render_step_kernel(RenderArgs a) {
     const float t0c = act ? a.t0[s] : 0.f, t1c = act ? a.t1[s] : 1.f;
     f.ts = (t0c * dcn) / dkn;
     f.te = (t1c * dcn) / dkn;
-    f.c = sigmoidf_(f.fs * inv_s);
-    f.e = sigmoidf_(f.fe * inv_s);
-    f.r = ((f.c - f.e) + 1e-5f) / (f.c + 1e-5f);
-    f.alpha = fminf(fmaxf(f.r, 0.f), 1.f);
     if (ad) {
       for (int c = 0; c < 3; ++c) f.g[c] = act ? a.grad_s[((int64_t)s * P + k) * 3 + c] : 0.f;
       f.proj[0] = f.proj[1] = f.proj[2] = 0.f;
@@ -183,10 +279,11 @@ render_step_kernel(RenderArgs a) {
   for (int j = 0; j < max_cnt; ++j) {
     const bool act = lane_ok && j < cnt;
     SampleF f = eval(j, act);
+    const Opacity<kFine> op(f.fs, f.fe, inv_s, act);
     if (act) {
-      const float w = f.alpha * T;
+      const float w = op.alpha * T;
       a.g_sdf_s[(int64_t)(base + j) * P + k] = T;  // parked for the reverse pass
-      T *= (1.f - f.alpha);
+      T *= op.om;
       ws += w;
       for (int c = 0; c < 3; ++c) cn[c] += w * f.g[c];
       const float nrm = sqrtf(f.g[0] * f.g[0] + f.g[1] * f.g[1] + f.g[2] * f.g[2]);
@@ -207,43 +304,40 @@ render_step_kernel(RenderArgs a) {
       }
     }
     l_n /= mask_sum;
-    const float lo = 1e-5f, hi = 1.f - 1e-5f;
-    const float xw = fminf(fmaxf(ws, lo), hi);
-    l_m = -(m * fmaxf(logf(xw), -100.f) + (1.f - m) * fmaxf(logf(1.f - xw), -100.f)) / n_mask;
-    const bool pass = ws >= lo && ws <= hi;
-    g_ws = pass ? a.mask_w * (xw - m) / fmaxf((1.f - xw) * xw, 1e-12f) / n_mask : 0.f;
+    const MaskLoss ml = mask_loss<kFine>(ws, T, m, a.mask_w, n_mask);
+    l_m = ml.l;
+    g_ws = ml.g;
     if (a.weight_sum) a.weight_sum[p * P + k] = ws;
     if (a.comp_normal)
       for (int c = 0; c < 3; ++c) a.comp_normal[(p * P + k) * 3 + c] = cn[c];
   }
   // ---------------- reverse ----------------
+  const float g_end = kFine ? g_ws * T : 0.f, g_rec = kFine ? 0.f : g_ws;
   float Q = 0.f, carry = 0.f, g_inv = 0.f;
-  float a_next = 0.f, gw_next = 0.f;  // alpha and dL/dw of sample j+1
+  float a_next = 0.f, om_next = 1.f, gw_next = 0.f;  // alpha, 1 - alpha and dL/dw of sample j+1
   for (int j = max_cnt - 1; j >= 0; --j) {
     const bool act = lane_ok && j < cnt;
     SampleF f = eval(j, act);
     const int s = base + j;
     const float Tj = act ? a.g_sdf_s[(int64_t)s * P + k] : 0.f;
-    const float w = f.alpha * Tj;
+    const Opacity<kFine> op(f.fs, f.fe, inv_s, act);
+    const float w = op.alpha * Tj;
     // dL/dgrad of this sample
     const float nrm = sqrtf(f.g[0] * f.g[0] + f.g[1] * f.g[1] + f.g[2] * f.g[2]);
     float gg[3];
     const float ek = nrm > 0.f ? a.eik_w * 2.f * (nrm - 1.f) / n_eik / nrm : 0.f;
     for (int c = 0; c < 3; ++c) gg[c] = act ? (w * g_cn[c] + ek * f.g[c]) : 0.f;
     // dL/dw and the weight recurrence
-    const float gw = act ? (g_ws + g_cn[0] * f.g[0] + g_cn[1] * f.g[1] + g_cn[2] * f.g[2]) : 0.f;
-    Q = (j == cnt - 1) ? 0.f : (gw_next * a_next) + (1.f - a_next) * Q;
-    const float g_alpha = act ? Tj * (gw - Q) : 0.f;
-    a_next = f.alpha;
+    const float gw = act ? (g_rec + g_cn[0] * f.g[0] + g_cn[1] * f.g[1] + g_cn[2] * f.g[2]) : 0.f;
+    Q = (j == cnt - 1) ? 0.f : (gw_next * a_next) + om_next * Q;
+    float g_alpha = act ? Tj * (gw - Q) : 0.f;
+    if (kFine && act && g_end != 0.f) g_alpha += g_end / op.om;
+    a_next = op.alpha;
+    om_next = op.om;
     gw_next = gw;
-    // alpha = clip(r): r = (c - e + eps) / (c + eps)
-    const float gr = (f.r >= 0.f && f.r <= 1.f) ? g_alpha : 0.f;
-    const float den = f.c + 1e-5f;
-    const float g_c = gr * f.e / (den * den);
-    const float g_e = -gr / den;
-    float g_fs = g_c * inv_s * f.c * (1.f - f.c);
-    float g_fe = g_e * inv_s * f.e * (1.f - f.e);
-    g_inv += act ? (g_c * f.fs * f.c * (1.f - f.c) + g_e * f.fe * f.e * (1.f - f.e)) : 0.f;
+    float g_fs, g_fe, gi;
+    op.grad(g_alpha, f.fs, f.fe, inv_s, g_fs, g_fe, gi);
+    g_inv += act ? gi : 0.f;
     if (ad) {
       if (act)
         for (int c = 0; c < 3; ++c) a.g_grad_s[((int64_t)s * P + k) * 3 + c] = gg[c];
@@ -313,12 +407,17 @@ render_step_kernel(RenderArgs a) {
 }
 
 // ---------------------------------------------------------------------------
-// Sample-parallel form for small patches (Ph x Pw <= 9): one wavefront per
-// patch, lane j = sample j of the patch (in chunks of 64), every ray of the
-// patch in the lane's registers, so the finite differences across the patch
-// are register arithmetic.  Along the samples, the transmittance is an
+// Sample-parallel form for small patches (Ph x Pw <= 9): one wavefront per row
+// of a patch, lane j = sample j of the patch (in chunks of 64), the row's rays
+// in the lane's registers, so the finite differences along a row are register
+// arithmetic; those across the rows read the neighbours' SDF values again and
+// exchange their gradients through LDS.  (The whole patch in one wavefront's
+// registers took 2 wavefronts per SIMD and their chains of scans nothing to run
+// beside: 3x3 patches, 1.2 M points in 2048 patches, 161 us, 110 so.)
+// Along the samples, the transmittance is an
 // exclusive prefix product and the weight backward's recurrence
 //   Q_j = gw_{j+1} alpha_{j+1} + (1 - alpha_{j+1}) Q_{j+1}
+// (gw: the normal loss's part of dL/dw)
 // a suffix scan of affine maps Q -> b + a Q, both as wavefront scans; chunks
 // carry T forwards and Q backwards.  The scans and sums are DPP lane moves
 // (VALU, no LDS round trip), the backward walks a chunk's samples in reverse
@@ -381,12 +480,18 @@ __device__ __forceinline__ void wave_incl_affine(float& a, float& b) {
   affine_step<0x143, 0xc>(a, b);
 }
 
-template <int Ph, int Pw, bool AD>
-__global__ void __launch_bounds__(64)
+template <int Ph, int Pw, bool AD, bool kFine>
+__global__ void __launch_bounds__(64 * Ph)
 render_patch_kernel(RenderArgs a) {
   constexpr int P = Ph * Pw;
+  __shared__ float sh_ay[AD ? 1 : 2][Ph][Pw][64];  // by chunk parity
+  __shared__ float sh_part[Ph][4];
   const int p = blockIdx.x;
   const int lane = threadIdx.x & 63;
+  // this wavefront's row of the patch and its neighbours (itself at the border)
+  const int row = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int up = row > 0 ? row - 1 : 0, dn = row < Ph - 1 ? row + 1 : Ph - 1;
+  const int k0 = row * Pw, ku = up * Pw, kd = dn * Pw;
   const float inv_s = *a.inv_s;
   const float mask_sum = *a.mask_sum;
   const int64_t n_s = *a.n_samples;
@@ -397,24 +502,14 @@ render_patch_kernel(RenderArgs a) {
   const int base = a.packed[2 * p], cnt = a.packed[2 * p + 1];
   constexpr int kc = (Ph / 2) * Pw + Pw / 2;
 
-  // per-ray constants of the patch
-  float o[P][3], d[P][3], dkn[P];
   const float* nn = a.plane_n + 3 * p;
-#pragma unroll
-  for (int k = 0; k < P; ++k) {
-#pragma unroll
-    for (int c = 0; c < 3; ++c) {
-      o[k][c] = a.rays_o[((int64_t)p * P + k) * 3 + c];
-      d[k][c] = a.rays_d[((int64_t)p * P + k) * 3 + c];
-    }
-    dkn[k] = (d[k][0] * nn[0] + d[k][1] * nn[1]) + d[k][2] * nn[2];
-  }
-  const float dcn = (d[kc][0] * nn[0] + d[kc][1] * nn[1]) + d[kc][2] * nn[2];
+  auto slope = [&](const float* d) { return (d[0] * nn[0] + d[1] * nn[1]) + d[2] * nn[2]; };
+  const float dcn = slope(a.rays_d + ((int64_t)p * P + kc) * 3);
 
-  // per-sample forward quantities of every ray (lane = sample j)
+  // per-sample forward quantities of the row's rays (lane = sample j)
   struct Q {
-    float fs[P], fe[P], c[P], e[P], r[P], alpha[P], g[P][3];
-    float gp_coef[P][3];  // dfd: 1/dtd, 1/denx, 1/deny of each ray
+    float fs[Pw], fe[Pw], g[Pw][3];
+    float gp_coef[Pw][3];  // dfd: dtd, denx, deny of each ray
   };
   auto eval = [&](int j, bool act, Q& q) {
     const int64_t s = (int64_t)base + j;
@@ -425,69 +520,82 @@ render_patch_kernel(RenderArgs a) {
       t0c = a.t0[s];
       t1c = a.t1[s];
     }
+    float fu[Pw], fd[Pw];
 #pragma unroll
-    for (int k = 0; k < P; ++k) {
+    for (int c = 0; c < Pw; ++c) {
       float fs = 0.f, fe = 0.f;
+      fu[c] = fd[c] = 0.f;
       if (act) {
-        fs = a.sdf_s[s * P + k];
-        fe = di >= 0 ? sdf_e[(int64_t)di * P + k] : a.sdf_s[(s + 1) * P + k];
+        fs = a.sdf_s[s * P + k0 + c];
+        fe = di >= 0 ? sdf_e[(int64_t)di * P + k0 + c] : a.sdf_s[(s + 1) * P + k0 + c];
+        if (!AD) {
+          fu[c] = a.sdf_s[s * P + ku + c];
+          fd[c] = a.sdf_s[s * P + kd + c];
+        }
       }
-      q.fs[k] = fs;
-      q.fe[k] = fe;
-      q.c[k] = sigmoidf_(fs * inv_s);
-      q.e[k] = sigmoidf_(fe * inv_s);
-      q.r[k] = ((q.c[k] - q.e[k]) + 1e-5f) / (q.c[k] + 1e-5f);
-      q.alpha[k] = act ? fminf(fmaxf(q.r[k], 0.f), 1.f) : 0.f;
+      q.fs[c] = fs;
+      q.fe[c] = fe;
     }
     if (AD) {
 #pragma unroll
-      for (int k = 0; k < P; ++k)
+      for (int k = 0; k < Pw; ++k)
 #pragma unroll
-        for (int c = 0; c < 3; ++c) q.g[k][c] = act ? a.grad_s[(s * P + k) * 3 + c] : 0.f;
+        for (int c = 0; c < 3; ++c) q.g[k][c] = act ? a.grad_s[(s * P + k0 + k) * 3 + c] : 0.f;
     } else {
-      float ts[P], te[P], x[P][3];
+      struct Pos {
+        float v[3];
+      };
+      float dtd[Pw];
+      auto pos = [&](int k, float& t, float& dk) {
+        const float* d = a.rays_d + ((int64_t)p * P + k) * 3;
+        const float* o = a.rays_o + ((int64_t)p * P + k) * 3;
+        dk = slope(d);
+        t = (t0c * dcn) / dk;
+        Pos x;
 #pragma unroll
-      for (int k = 0; k < P; ++k) {
-        ts[k] = (t0c * dcn) / dkn[k];
-        te[k] = (t1c * dcn) / dkn[k];
-#pragma unroll
-        for (int c = 0; c < 3; ++c) x[k][c] = o[k][c] + d[k][c] * ts[k];
-      }
-      auto dist = [&](int k1, int k2) {
-        const float dx = x[k2][0] - x[k1][0], dy = x[k2][1] - x[k1][1], dz = x[k2][2] - x[k1][2];
+        for (int c = 0; c < 3; ++c) x.v[c] = o[c] + d[c] * t;
+        return x;
+      };
+      auto dist = [&](const Pos& x1, const Pos& x2) {
+        const float dx = x2.v[0] - x1.v[0], dy = x2.v[1] - x1.v[1], dz = x2.v[2] - x1.v[2];
         return sqrtf(dx * dx + dy * dy + dz * dz);
       };
+      Pos x[Pw];
+      float deny[Pw];
 #pragma unroll
-      for (int k = 0; k < P; ++k) {
-        const int row = k / Pw, col = k % Pw;
-        const float dtd = te[k] - ts[k];
-        const float df_dt = (q.fe[k] - q.fs[k]) / dtd;
-        float denx, dfx, deny, dfy;
-        if (col == 0) { denx = dist(k, k + 1); dfx = (q.fs[k + 1] - q.fs[k]) / denx; }
-        else if (col == Pw - 1) { denx = dist(k - 1, k); dfx = (q.fs[k] - q.fs[k - 1]) / denx; }
-        else { denx = dist(k - 1, k) + dist(k, k + 1); dfx = (q.fs[k + 1] - q.fs[k - 1]) / denx; }
-        if (row == 0) { deny = dist(k, k + Pw); dfy = (q.fs[k + Pw] - q.fs[k]) / deny; }
-        else if (row == Ph - 1) { deny = dist(k - Pw, k); dfy = (q.fs[k] - q.fs[k - Pw]) / deny; }
-        else { deny = dist(k - Pw, k) + dist(k, k + Pw); dfy = (q.fs[k + Pw] - q.fs[k - Pw]) / deny; }
-        q.gp_coef[k][0] = dtd;
-        q.gp_coef[k][1] = denx;
-        q.gp_coef[k][2] = deny;
-        const float* vi = a.vinv + ((int64_t)p * P + k) * 9;
+      for (int c = 0; c < Pw; ++c) {
+        float ts, dk, t_, d_;
+        x[c] = pos(k0 + c, ts, dk);
+        dtd[c] = (t1c * dcn) / dk - ts;
+        const Pos xu = pos(ku + c, t_, d_), xd = pos(kd + c, t_, d_);
+        deny[c] = dist(xu, x[c]) + dist(x[c], xd);  // (a border row's own distance is 0)
+      }
+#pragma unroll
+      for (int col = 0; col < Pw; ++col) {
+        const float df_dt = (q.fe[col] - q.fs[col]) / dtd[col];
+        float denx, dfx;
+        if (col == 0) { denx = dist(x[0], x[1]); dfx = (q.fs[1] - q.fs[0]) / denx; }
+        else if (col == Pw - 1) { denx = dist(x[col - 1], x[col]); dfx = (q.fs[col] - q.fs[col - 1]) / denx; }
+        else { denx = dist(x[col - 1], x[col]) + dist(x[col], x[col + 1]); dfx = (q.fs[col + 1] - q.fs[col - 1]) / denx; }
+        const float dfy = (fd[col] - fu[col]) / deny[col];
+        q.gp_coef[col][0] = dtd[col];
+        q.gp_coef[col][1] = denx;
+        q.gp_coef[col][2] = deny[col];
+        const float* vi = a.vinv + ((int64_t)p * P + k0 + col) * 9;
 #pragma unroll
         for (int c = 0; c < 3; ++c)
-          q.g[k][c] = act ? (vi[3 * c + 0] * df_dt + vi[3 * c + 1] * dfx + vi[3 * c + 2] * dfy) : 0.f;
+          q.g[col][c] = act ? (vi[3 * c + 0] * df_dt + vi[3 * c + 1] * dfx + vi[3 * c + 2] * dfy) : 0.f;
       }
     }
   };
 
   // ---------------- forward: T by prefix products, sums over samples --------
-  float Tin[P], ws[P], cn[P][3], eik[P];
+  float Tin[Pw], ws[Pw], cn[Pw][3], eik = 0.f;
 #pragma unroll
-  for (int k = 0; k < P; ++k) {
+  for (int k = 0; k < Pw; ++k) {
     Tin[k] = 1.f;
     ws[k] = 0.f;
     cn[k][0] = cn[k][1] = cn[k][2] = 0.f;
-    eik[k] = 0.f;
   }
   for (int j0 = 0; j0 < cnt; j0 += 64) {
     const int j = j0 + lane;
@@ -495,39 +603,41 @@ render_patch_kernel(RenderArgs a) {
     Q q;
     eval(j, act, q);
 #pragma unroll
-    for (int k = 0; k < P; ++k) {
+    for (int k = 0; k < Pw; ++k) {
+      const Opacity<kFine> op(q.fs[k], q.fe[k], inv_s, act);
       // inclusive prefix product of (1 - alpha), then exclusive (wave_shr:1)
-      const float incl = wave_incl_prod(1.f - q.alpha[k]);
+      const float incl = wave_incl_prod(op.om);
       const float excl = dpp_or<0x138>(1.f, incl);
       const float T = Tin[k] * excl;
-      const float w = q.alpha[k] * T;
-      if (act) a.g_sdf_s[((int64_t)base + j) * P + k] = T;  // parked for the backward
+      const float w = op.alpha * T;
+      if (act) a.g_sdf_s[((int64_t)base + j) * P + k0 + k] = T;  // parked for the backward
       const float nrm = sqrtf(q.g[k][0] * q.g[k][0] + q.g[k][1] * q.g[k][1] + q.g[k][2] * q.g[k][2]);
       // per-lane partial sums, reduced once after the last chunk
       ws[k] += w;
 #pragma unroll
       for (int c = 0; c < 3; ++c) cn[k][c] += w * q.g[k][c];
-      eik[k] += act ? (nrm - 1.f) * (nrm - 1.f) : 0.f;
+      eik += act ? (nrm - 1.f) * (nrm - 1.f) : 0.f;
       Tin[k] *= lane63(incl);
     }
   }
 #pragma unroll
-  for (int k = 0; k < P; ++k) {
+  for (int k = 0; k < Pw; ++k) {
     ws[k] = wave_sum(ws[k]);
 #pragma unroll
     for (int c = 0; c < 3; ++c) cn[k][c] = wave_sum(cn[k][c]);
-    eik[k] = wave_sum(eik[k]);
   }
+  const float l_e = wave_sum(eik) / n_eik;
   // ---------------- losses of every ray and their gradients -----------------
-  float g_cn[P][3], g_ws[P];
-  float l_n = 0.f, l_m = 0.f, l_e = 0.f;
+  float g_cn[Pw][3], g_ws[Pw];  // fine: g_ws T_end
+  float l_n = 0.f, l_m = 0.f;
 #pragma unroll
-  for (int k = 0; k < P; ++k) {
-    const float m = a.mask[(int64_t)p * P + k];
+  for (int k = 0; k < Pw; ++k) {
+    const int64_t ray = (int64_t)p * P + k0 + k;
+    const float m = a.mask[ray];
     float ln = 0.f;
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
-      const float nt = a.n_true[((int64_t)p * P + k) * 3 + c];
+      const float nt = a.n_true[ray * 3 + c];
       const float err = (cn[k][c] - nt) * m;
       if (a.l1) {
         ln += fabsf(err);
@@ -538,25 +648,22 @@ render_patch_kernel(RenderArgs a) {
       }
     }
     l_n += ln / mask_sum;
-    const float lo = 1e-5f, hi = 1.f - 1e-5f;
-    const float xw = fminf(fmaxf(ws[k], lo), hi);
-    l_m += -(m * fmaxf(logf(xw), -100.f) + (1.f - m) * fmaxf(logf(1.f - xw), -100.f)) / n_mask;
-    const bool pass = ws[k] >= lo && ws[k] <= hi;
-    g_ws[k] = pass ? a.mask_w * (xw - m) / fmaxf((1.f - xw) * xw, 1e-12f) / n_mask : 0.f;
-    l_e += eik[k] / n_eik;
+    const MaskLoss ml = mask_loss<kFine>(ws[k], Tin[k], m, a.mask_w, n_mask);
+    l_m += ml.l;
+    g_ws[k] = kFine ? ml.g * Tin[k] : ml.g;
     if (lane == 0) {
-      if (a.weight_sum) a.weight_sum[(int64_t)p * P + k] = ws[k];
+      if (a.weight_sum) a.weight_sum[ray] = ws[k];
       if (a.comp_normal)
 #pragma unroll
-        for (int c = 0; c < 3; ++c) a.comp_normal[((int64_t)p * P + k) * 3 + c] = cn[k][c];
+        for (int c = 0; c < 3; ++c) a.comp_normal[ray * 3 + c] = cn[k][c];
     }
   }
   // ---------------- backward, chunks in reverse ------------------------------
-  float Qin[P];
+  float Qin[Pw];
 #pragma unroll
-  for (int k = 0; k < P; ++k) Qin[k] = 0.f;
+  for (int k = 0; k < Pw; ++k) Qin[k] = 0.f;
   float g_inv = 0.f;
-  const int n_chunks = (cnt + 63) / 64;
+  const int n_chunks = (cnt + 63) / 64;  // the same for every wavefront of the patch
   for (int ch = n_chunks - 1; ch >= 0; --ch) {
     // reverse lane order: lane 0 holds the chunk's last sample
     const int j = ch * 64 + 63 - lane;
@@ -565,68 +672,73 @@ render_patch_kernel(RenderArgs a) {
     Q q;
     eval(j, act, q);
     const int di = act ? a.diff_idx[s] : 0;
-    float G[P];  // dL/dfs of every ray of this sample (own terms + neighbours')
-    float GE[P]; // dL/dfe
+    float G[Pw];   // dL/dfs of the row's rays of this sample (own terms + neighbours')
+    float GE[Pw];  // dL/dfe
+    float ax[Pw];
 #pragma unroll
-    for (int k = 0; k < P; ++k) {
-      const float Tj = act ? a.g_sdf_s[s * P + k] : 0.f;
-      const float w = q.alpha[k] * Tj;
+    for (int k = 0; k < Pw; ++k) {
+      const Opacity<kFine> op(q.fs[k], q.fe[k], inv_s, act);
+      const float Tj = act ? a.g_sdf_s[s * P + k0 + k] : 0.f;
+      const float w = op.alpha * Tj;
       const float nrm = sqrtf(q.g[k][0] * q.g[k][0] + q.g[k][1] * q.g[k][1] + q.g[k][2] * q.g[k][2]);
       const float ek = nrm > 0.f ? a.eik_w * 2.f * (nrm - 1.f) / n_eik / nrm : 0.f;
       float gg[3];
 #pragma unroll
       for (int c = 0; c < 3; ++c) gg[c] = act ? (w * g_cn[k][c] + ek * q.g[k][c]) : 0.f;
-      const float gw = act ? (g_ws[k] + g_cn[k][0] * q.g[k][0] + g_cn[k][1] * q.g[k][1] +
-                              g_cn[k][2] * q.g[k][2]) : 0.f;
+      const float gw = act ? ((kFine ? 0.f : g_ws[k]) + g_cn[k][0] * q.g[k][0] +
+                              g_cn[k][1] * q.g[k][1] + g_cn[k][2] * q.g[k][2]) : 0.f;
       // suffix scan of the maps M_j(Q) = gw_j alpha_j + (1 - alpha_j) Q: in
       // reversed lane order a prefix scan, lane l = S_j (chunk end .. j)
-      float ma = act ? 1.f - q.alpha[k] : 1.f, mb = act ? gw * q.alpha[k] : 0.f;
+      float ma = op.om, mb = gw * op.alpha;
       wave_incl_affine(ma, mb);
       // Q_j = S_{j+1}(Qin): the previous lane's map (lane 0: the identity)
       const float sa = dpp_or<0x138>(1.f, ma), sb = dpp_or<0x138>(0.f, mb);
       const float Qj = sb + sa * Qin[k];
       const float Qnext = lane63(mb + ma * Qin[k]);  // S_{chunk start}(Qin): carried back
-      const float g_alpha = act ? Tj * (gw - Qj) : 0.f;
-      const float gr = (q.r[k] >= 0.f && q.r[k] <= 1.f) ? g_alpha : 0.f;
-      const float den = q.c[k] + 1e-5f;
-      const float g_c = gr * q.e[k] / (den * den);
-      const float g_e = -gr / den;
-      G[k] = g_c * inv_s * q.c[k] * (1.f - q.c[k]);
-      GE[k] = g_e * inv_s * q.e[k] * (1.f - q.e[k]);
-      g_inv += act ? (g_c * q.fs[k] * q.c[k] * (1.f - q.c[k]) + g_e * q.fe[k] * q.e[k] * (1.f - q.e[k])) : 0.f;
+      float g_alpha = act ? Tj * (gw - Qj) : 0.f;
+      if (kFine && act && g_ws[k] != 0.f) g_alpha += g_ws[k] / op.om;
+      float gi;
+      op.grad(g_alpha, q.fs[k], q.fe[k], inv_s, G[k], GE[k], gi);
+      g_inv += act ? gi : 0.f;
       Qin[k] = Qnext;
       if (AD) {
         if (act)
 #pragma unroll
-          for (int c = 0; c < 3; ++c) a.g_grad_s[(s * P + k) * 3 + c] = gg[c];
+          for (int c = 0; c < 3; ++c) a.g_grad_s[(s * P + k0 + k) * 3 + c] = gg[c];
       } else {
-        const float* vi = a.vinv + ((int64_t)p * P + k) * 9;
-        // grad = V^-1 proj  =>  dL/dproj = V^-T dL/dgrad; kept in gg
+        const float* vi = a.vinv + ((int64_t)p * P + k0 + k) * 9;
+        // grad = V^-1 proj  =>  dL/dproj = V^-T dL/dgrad
         const float gp0 = vi[0] * gg[0] + vi[3] * gg[1] + vi[6] * gg[2];
         const float gp1 = vi[1] * gg[0] + vi[4] * gg[1] + vi[7] * gg[2];
         const float gp2 = vi[2] * gg[0] + vi[5] * gg[1] + vi[8] * gg[2];
-        gg[0] = gp0 / q.gp_coef[k][0];
-        gg[1] = act ? gp1 / q.gp_coef[k][1] : 0.f;
-        gg[2] = act ? gp2 / q.gp_coef[k][2] : 0.f;
-        q.gp_coef[k][0] = gg[0];
-        q.gp_coef[k][1] = gg[1];
-        q.gp_coef[k][2] = gg[2];
+        // df_dt = (fe - fs) / dtd
+        const float at = gp0 / q.gp_coef[k][0];
+        GE[k] += at;
+        G[k] -= at;
+        ax[k] = act ? gp1 / q.gp_coef[k][1] : 0.f;
+        sh_ay[ch & 1][row][k][lane] = act ? gp2 / q.gp_coef[k][2] : 0.f;
       }
     }
     if (!AD) {
-      // df_dt = (fe - fs) / dtd; finite differences across the patch
+      // finite differences along the row ...
 #pragma unroll
-      for (int k = 0; k < P; ++k) {
-        const int row = k / Pw, col = k % Pw;
-        GE[k] += q.gp_coef[k][0];
-        G[k] -= q.gp_coef[k][0];
-        const float ax = q.gp_coef[k][1], ay = q.gp_coef[k][2];
-        if (col == 0) { G[k + 1] += ax; G[k] -= ax; }
-        else if (col == Pw - 1) { G[k] += ax; G[k - 1] -= ax; }
-        else { G[k + 1] += ax; G[k - 1] -= ax; }
-        if (row == 0) { G[k + Pw] += ay; G[k] -= ay; }
-        else if (row == Ph - 1) { G[k] += ay; G[k - Pw] -= ay; }
-        else { G[k + Pw] += ay; G[k - Pw] -= ay; }
+      for (int col = 0; col < Pw; ++col) {
+        if (col == 0) { G[1] += ax[0]; G[0] -= ax[0]; }
+        else if (col == Pw - 1) { G[col] += ax[col]; G[col - 1] -= ax[col]; }
+        else { G[col + 1] += ax[col]; G[col - 1] -= ax[col]; }
+      }
+      // ... and across the rows: row r's goes to the row below it (+) and the
+      // row above it (-), to itself at the border.  (One barrier a chunk: a
+      // half is written again two chunks later, behind the next one's barrier.)
+      __syncthreads();
+      for (int r = up; r <= dn; ++r) {
+        const bool plus = (r < Ph - 1 ? r + 1 : r) == row, minus = (r > 0 ? r - 1 : r) == row;
+        if (plus)
+#pragma unroll
+          for (int k = 0; k < Pw; ++k) G[k] += sh_ay[ch & 1][r][k][lane];
+        if (minus)
+#pragma unroll
+          for (int k = 0; k < Pw; ++k) G[k] -= sh_ay[ch & 1][r][k][lane];
       }
     }
     // ends: own SDF row, or the next sample's start (added to that start);
@@ -634,31 +746,37 @@ render_patch_kernel(RenderArgs a) {
     const bool to_next = act && di < 0;
     const float prev_to_next = dpp_or<0x130>(0.f, to_next ? 1.f : 0.f);
 #pragma unroll
-    for (int k = 0; k < P; ++k) {
+    for (int k = 0; k < Pw; ++k) {
       const float from_prev = dpp_or<0x130>(0.f, GE[k]);
       float gs = G[k];
       if (lane < 63 && prev_to_next != 0.f) gs += from_prev;
       if (act) {
         // the chunk's first sample may also receive from the previous chunk,
         // whose lane 63 adds its share later (read-modify-write below)
-        a.g_sdf_s[s * P + k] = gs;
-        if (di >= 0) g_sdf_e[(int64_t)di * P + k] = GE[k];
+        a.g_sdf_s[s * P + k0 + k] = gs;
+        if (di >= 0) g_sdf_e[(int64_t)di * P + k0 + k] = GE[k];
       }
     }
     if (lane == 0 && to_next && j + 1 < cnt) {
       // sample j + 1 is the next chunk's first sample, already written
 #pragma unroll
-      for (int k = 0; k < P; ++k) a.g_sdf_s[(s + 1) * P + k] += GE[k];
+      for (int k = 0; k < Pw; ++k) a.g_sdf_s[(s + 1) * P + k0 + k] += GE[k];
     }
   }
-  // per-patch partials: normal, mask, eikonal, dL/dinv_s
+  // per-patch partials: normal, mask, eikonal, dL/dinv_s, the rows in order
   const float v3 = wave_sum(g_inv);
   if (lane == 0) {
-    float* o4 = a.partials + 4 * (int64_t)p;
-    o4[0] = a.normal_w * l_n;
-    o4[1] = a.mask_w * l_m;
-    o4[2] = a.eik_w * l_e;
-    o4[3] = v3;
+    sh_part[row][0] = a.normal_w * l_n;
+    sh_part[row][1] = a.mask_w * l_m;
+    sh_part[row][2] = a.eik_w * l_e;
+    sh_part[row][3] = v3;
+  }
+  __syncthreads();
+  if (threadIdx.x < 4) {
+    float t = 0.f;
+#pragma unroll
+    for (int r = 0; r < Ph; ++r) t += sh_part[r][threadIdx.x];
+    a.partials[4 * (int64_t)p + threadIdx.x] = t;
   }
 }
 
@@ -687,25 +805,17 @@ static int g_render_impl = 1;  // 1: sample-parallel kernel where the patch shap
 
 using namespace sn;
 
-extern "C" {
-
-int sn_render_step_waves(int32_t n_patches, int32_t patch_size) {
-  if (patch_size <= 0 || patch_size > 64 || n_patches < 0) return -1;
-  return n_patches;  // one partial row per patch at most (sample-parallel kernel)
-}
-
-void sn_render_step_set_impl(int32_t impl) { g_render_impl = impl; }
-
-int sn_render_step(int32_t n_patches, int32_t patch_h, int32_t patch_w, const float* rays_o,
-                   const float* rays_d, const float* plane_n, const float* v_inv,
-                   const float* n_true, const float* mask, const int32_t* packed_info,
-                   const float* t_starts, const float* t_ends, const int32_t* diff_idx,
-                   const float* sdf_starts, const float* sdf_ends, const float* grad_starts,
-                   const float* inv_s, const float* mask_sum, const int32_t* n_samples,
-                   float normal_w, float eik_w, float mask_w, int32_t loss_l1,
-                   float* g_sdf_starts, float* g_sdf_ends, float* g_grad_starts,
-                   float* losses, float* partials, float* weight_sum, float* comp_normal,
-                   void* stream) {
+template <bool kFine>
+static int render_step_impl(int32_t n_patches, int32_t patch_h, int32_t patch_w, const float* rays_o,
+                            const float* rays_d, const float* plane_n, const float* v_inv,
+                            const float* n_true, const float* mask, const int32_t* packed_info,
+                            const float* t_starts, const float* t_ends, const int32_t* diff_idx,
+                            const float* sdf_starts, const float* sdf_ends, const float* grad_starts,
+                            const float* inv_s, const float* mask_sum, const int32_t* n_samples,
+                            float normal_w, float eik_w, float mask_w, int32_t loss_l1,
+                            float* g_sdf_starts, float* g_sdf_ends, float* g_grad_starts,
+                            float* losses, float* partials, float* weight_sum, float* comp_normal,
+                            void* stream) {
   clear_error();
   const int P = patch_h * patch_w;
   SN_REQUIRE(n_patches >= 0 && patch_h > 0 && patch_w > 0 && P <= 64,
@@ -752,19 +862,62 @@ int sn_render_step(int32_t n_patches, int32_t patch_h, int32_t patch_w, const fl
   hipStream_t s = as_stream(stream);
   const bool ad = grad_starts != nullptr;
   if (g_render_impl == 1 && patch_h == 3 && patch_w == 3) {
-    if (ad) render_patch_kernel<3, 3, true><<<n_patches, 64, 0, s>>>(a);
-    else render_patch_kernel<3, 3, false><<<n_patches, 64, 0, s>>>(a);
+    if (ad) render_patch_kernel<3, 3, true, kFine><<<n_patches, 64 * 3, 0, s>>>(a);
+    else render_patch_kernel<3, 3, false, kFine><<<n_patches, 64 * 3, 0, s>>>(a);
     reduce4_wide_kernel<<<1, 256, 0, s>>>(partials, n_patches, losses);
   } else if (g_render_impl == 1 && patch_h == 2 && patch_w == 4) {
-    if (ad) render_patch_kernel<2, 4, true><<<n_patches, 64, 0, s>>>(a);
-    else render_patch_kernel<2, 4, false><<<n_patches, 64, 0, s>>>(a);
+    if (ad) render_patch_kernel<2, 4, true, kFine><<<n_patches, 64 * 2, 0, s>>>(a);
+    else render_patch_kernel<2, 4, false, kFine><<<n_patches, 64 * 2, 0, s>>>(a);
     reduce4_wide_kernel<<<1, 256, 0, s>>>(partials, n_patches, losses);
   } else {
     const int waves = (int)ceil_div(n_patches, 64 / P);
-    render_step_kernel<<<waves, 64, 0, s>>>(a);
+    render_step_kernel<kFine><<<waves, 64, 0, s>>>(a);
     reduce4_wide_kernel<<<1, 256, 0, s>>>(partials, waves, losses);
   }
   return check_launch("sn_render_step");
+}
+
+extern "C" {
+
+int sn_render_step_waves(int32_t n_patches, int32_t patch_size) {
+  if (patch_size <= 0 || patch_size > 64 || n_patches < 0) return -1;
+  return n_patches;  // one partial row per patch at most (sample-parallel kernel)
+}
+
+void sn_render_step_set_impl(int32_t impl) { g_render_impl = impl; }
+
+int sn_render_step(int32_t n_patches, int32_t patch_h, int32_t patch_w, const float* rays_o,
+                   const float* rays_d, const float* plane_n, const float* v_inv,
+                   const float* n_true, const float* mask, const int32_t* packed_info,
+                   const float* t_starts, const float* t_ends, const int32_t* diff_idx,
+                   const float* sdf_starts, const float* sdf_ends, const float* grad_starts,
+                   const float* inv_s, const float* mask_sum, const int32_t* n_samples,
+                   float normal_w, float eik_w, float mask_w, int32_t loss_l1,
+                   float* g_sdf_starts, float* g_sdf_ends, float* g_grad_starts,
+                   float* losses, float* partials, float* weight_sum, float* comp_normal,
+                   void* stream) {
+  return render_step_impl<false>(
+      n_patches, patch_h, patch_w, rays_o, rays_d, plane_n, v_inv, n_true, mask,
+      packed_info, t_starts, t_ends, diff_idx, sdf_starts, sdf_ends, grad_starts, inv_s,
+      mask_sum, n_samples, normal_w, eik_w, mask_w, loss_l1, g_sdf_starts, g_sdf_ends,
+      g_grad_starts, losses, partials, weight_sum, comp_normal, stream);
+}
+
+int sn_render_step_fine(int32_t n_patches, int32_t patch_h, int32_t patch_w, const float* rays_o,
+                        const float* rays_d, const float* plane_n, const float* v_inv,
+                        const float* n_true, const float* mask, const int32_t* packed_info,
+                        const float* t_starts, const float* t_ends, const int32_t* diff_idx,
+                        const float* sdf_starts, const float* sdf_ends, const float* grad_starts,
+                        const float* inv_s, const float* mask_sum, const int32_t* n_samples,
+                        float normal_w, float eik_w, float mask_w, int32_t loss_l1,
+                        float* g_sdf_starts, float* g_sdf_ends, float* g_grad_starts,
+                        float* losses, float* partials, float* weight_sum, float* comp_normal,
+                        void* stream) {
+  return render_step_impl<true>(
+      n_patches, patch_h, patch_w, rays_o, rays_d, plane_n, v_inv, n_true, mask,
+      packed_info, t_starts, t_ends, diff_idx, sdf_starts, sdf_ends, grad_starts, inv_s,
+      mask_sum, n_samples, normal_w, eik_w, mask_w, loss_l1, g_sdf_starts, g_sdf_ends,
+      g_grad_starts, losses, partials, weight_sum, comp_normal, stream);
 }
 
 }  // extern "C"

@@ -94,7 +94,9 @@ class _RenderStepFn(torch.autograd.Function):
         waves = _lib.lib().sn_render_step_waves(st["B"], P)
         partials = torch.empty(4 * waves, device=dev)
         se = sdf_e if Nd else torch.zeros(P, device=dev)
-        call("sn_render_step", st["B"], st["Ph"], st["Pw"], ptr(st["rays_o"]), ptr(st["rays_d"]),
+        # (the fine form pays where the SDF is of fp32 accuracy)
+        call("sn_render_step_fine" if st["fine"] else "sn_render_step", st["B"], st["Ph"],
+             st["Pw"], ptr(st["rays_o"]), ptr(st["rays_d"]),
              ptr(st["plane_n"]), ptr(st["v_inv"]), ptr(st["n_true"]), ptr(st["mask"]),
              ptr(st["packed"]), ptr(st["t0"]), ptr(st["t1"]), ptr(st["diff_idx"]),
              ptr(sdf_s), ptr(se), ptr(grad_s if st["ad"] else None), ptr(inv_s),
@@ -216,6 +218,7 @@ class FusedStep:
             grad_s = None
         mask_b = (mask > 0.5).float() if self.mask_w > 0 else torch.ones_like(mask)
         st = dict(B=B, Ph=Ph, Pw=Pw, P=P, S=S, Nd=Nd, ad=self.method == "ad",
+                  fine=getattr(net, "mlp_precision", "fp32") != "fp16",
                   rays_o=rays_o.contiguous(), rays_d=rays_d.contiguous(),
                   plane_n=plane_n.contiguous(), v_inv=v_inv.contiguous(),
                   n_true=n_true.contiguous(), mask=mask_b.reshape(B, P).contiguous(),

@@ -423,7 +423,9 @@ class SyncFreeStep:
         else:
             self._sdf_fwd(self.pts, self.enc, self.sdf, c1, self.ne, mlp_d, s)
         ad = self.ad
-        call("sn_render_step", B, self.Ph, self.Pw, ptr(self.rays_o), ptr(self.rays_d),
+        # (the fine form pays where the SDF is of fp32 accuracy)
+        render = "sn_render_step" if self.precision == "fp16" else "sn_render_step_fine"
+        call(render, B, self.Ph, self.Pw, ptr(self.rays_o), ptr(self.rays_d),
              ptr(self.plane_n), ptr(self.v_inv), ptr(self.n_true), ptr(self.mask),
              ptr(self.packed), ptr(self.t0), ptr(self.t1), ptr(self.didx), ptr(self.sdf), None,
              ptr(self.grad_pts) if ad else None, ptr(self.inv_s), ptr(self.mask_sum),
