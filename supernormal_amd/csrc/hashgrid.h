@@ -38,6 +38,50 @@ int64_t make_hashgrid_desc(int32_t n_levels, int32_t log2_T, int32_t base_res,
                            float per_level_scale, int32_t n_active, HashGridDesc* d);
 
 #ifdef __HIPCC__
+// Table rows of the 8 corners (order c = bx | by<<1 | bz<<2) of the cell with
+// integer coordinates g.  One uniform branch per level; the hash's products
+// are formed once per axis, and a dense level's rows from the first corner's:
+// its row number is reduced modulo the level size once (only where some row
+// number reaches it: cells of negative coordinates wrap through uint32), and a
+// corner `off` rows further (off < size) is that remainder + off, less the
+// size at most once -- or, where the uint32 sum wraps, the small wrapped
+// number itself.  (A modulo per corner with its branches had made the corner
+// indices a third of the gather and record kernels' instructions.)
+__device__ __forceinline__ void hg_rows(const uint32_t g[3], uint32_t res, uint32_t hs, bool dense,
+                                        uint32_t idx[8]) {
+  if (dense) {  // uniform
+    const uint32_t rr = res * res;
+    const uint32_t base = g[0] + g[1] * res + g[2] * rr;
+    const uint32_t far = 1u + res + rr;  // the last corner's offset
+    if (base + far < base || base + far >= hs) {
+      const uint32_t m = base % hs;
+#pragma unroll
+      for (int c = 0; c < 8; ++c) {
+        const uint32_t off = (c & 1) + ((c >> 1) & 1) * res + ((c >> 2) & 1) * rr;
+        const uint32_t id = base + off, t = m + off;
+        idx[c] = id < base ? id : (t < hs ? t : t - hs);
+      }
+      // (levels of fewer rows than a corner's offset: the plain form)
+      if (far >= hs) {
+#pragma unroll
+        for (int c = 0; c < 8; ++c)
+          idx[c] = (base + (c & 1) + ((c >> 1) & 1) * res + ((c >> 2) & 1) * rr) % hs;
+      }
+    } else {
+#pragma unroll
+      for (int c = 0; c < 8; ++c)
+        idx[c] = base + (c & 1) + ((c >> 1) & 1) * res + ((c >> 2) & 1) * rr;
+    }
+  } else {
+    const uint32_t y0 = g[1] * 2654435761u, z0 = g[2] * 805459861u;
+    const uint32_t y1 = y0 + 2654435761u, z1 = z0 + 805459861u, mask = hs - 1u;
+    const uint32_t x0 = g[0], x1 = g[0] + 1u;
+#pragma unroll
+    for (int c = 0; c < 8; ++c)
+      idx[c] = ((c & 1 ? x1 : x0) ^ ((c & 2 ? y1 : y0) ^ (c & 4 ? z1 : z0))) & mask;
+  }
+}
+
 // Corner indices/weights of one level.  frac in [0,1); w[c] in corner order
 // c = bx | by<<1 | bz<<2, computed as ((w_x) * w_y) * w_z like the reference loop;
 // g = the cell's integer coordinates (corner 0).
@@ -45,9 +89,6 @@ __device__ __forceinline__ void hg_level(const float x[3], const HashGridDesc& d
                                          uint32_t idx[8], float w[8], float frac[3],
                                          uint32_t g[3]) {
   const float sc = d.scale[l];
-  const uint32_t res = d.res[l];
-  const uint32_t hs = d.hsize[l];
-  const bool dense = (d.dense_mask >> l) & 1u;
 #pragma unroll
   for (int k = 0; k < 3; ++k) {
     float p = fmaf(sc, x[k], 0.5f);
@@ -55,17 +96,9 @@ __device__ __forceinline__ void hg_level(const float x[3], const HashGridDesc& d
     g[k] = (uint32_t)(int32_t)fl;
     frac[k] = p - fl;
   }
+  hg_rows(g, d.res[l], d.hsize[l], (d.dense_mask >> l) & 1u, idx);
 #pragma unroll
   for (int c = 0; c < 8; ++c) {
-    const uint32_t gx = g[0] + (c & 1), gy = g[1] + ((c >> 1) & 1), gz = g[2] + ((c >> 2) & 1);
-    uint32_t id;
-    if (dense) {
-      id = gx + gy * res + gz * res * res;
-      id = id < hs ? id : id % hs;
-    } else {
-      id = (gx ^ (gy * 2654435761u) ^ (gz * 805459861u)) & (hs - 1u);
-    }
-    idx[c] = id;
     float wt = (c & 1) ? frac[0] : 1.f - frac[0];
     wt *= ((c >> 1) & 1) ? frac[1] : 1.f - frac[1];
     wt *= ((c >> 2) & 1) ? frac[2] : 1.f - frac[2];

@@ -8,7 +8,9 @@
 // wavefront touches (coarse dense levels stay in L2; fine hashed levels are
 // random 8-byte gathers).  Parameter gradients are fp32 atomics, like the
 // reference's tcnn backward.
+#include <algorithm>
 #include <cmath>
+#include <type_traits>
 
 #include "hashgrid.h"
 #include "sn_common.h"
@@ -562,25 +564,30 @@ hash_bwd_lds_kernel(const float* __restrict__ x, int64_t n_cap, const int32_t* _
 // ---------------------------------------------------------------------------
 // Bucket path (with a workspace).  Two kernels, no fp32 atomics:
 //
-// 1. hash_bwd_rec_kernel: a workgroup takes kRecThreads (512) consecutive points and, per
-//    level, turns their corner contributions into records (table row, F
-//    values).  Lanes of a wavefront whose points lie in the same cell (common
-//    on coarse and middle levels: a wavefront holds neighbouring samples of
-//    a few rays of one patch) are summed first with cross-lane (DPP)
-//    reduce-scatters and leave one record per corner; the other lanes leave
-//    one record per corner each.
-//    Records go to the list of their bucket (kBucketEntries consecutive rows
-//    of the level): ranks within the workgroup come from integer LDS atomics,
+// 1. hash_bwd_rec_kernel: a workgroup takes kRecThreads (512) consecutive
+//    points and, per level, turns their corner contributions into records
+//    (table row, F values).  Lanes of a wavefront whose points lie in the same
+//    cell (common on coarse and middle levels: a wavefront holds neighbouring
+//    samples of a few rays of one patch) are summed first with cross-lane (DPP)
+//    reduce-scatters and leave their corners' records once; the other lanes
+//    leave theirs each.
+//    Records travel as x pairs (corners 2q and 2q + 1: one word of two 16-bit
+//    rows, 2F floats): x is the hash's and the dense index's fastest axis, so
+//    both rows lie in one bucket all but always, and ranks, staging and writes
+//    are paid once for two records.  A pair in two buckets leaves its second
+//    row in another pass over the level.
+//    Pairs go to the list of their bucket (kBucketEntries consecutive rows of
+//    the level): ranks within the workgroup come from integer LDS atomics,
 //    room in each list from one global atomic per (workgroup, level, bucket).
-//    Per level: ranks, barrier, offsets (one wavefront's scan, its
-//    reservation atomics issued first), barrier, staging in LDS by bucket
-//    while those atomics are in flight, barrier, coalesced writes (measured
-//    per level and workgroup on the late iterations of a full training run,
-//    with the reservation already overlapping the staging but before the
-//    per-wavefront level maximum and the DPP scan: hashing and loads 1.1 us,
-//    group search 1.6 us, ranks 1.35 us, waiting for the slowest wavefront
-//    1.4 us, scan 0.6 us, staging 0.6 us (wavefront 0 with the reservation
-//    1.4 us), writes 1.1 us).
+//    Two barriers a level, the levels overlapped: ranks of level l, barrier,
+//    reservation atomics of level l issued, the staged pairs of level l - 1
+//    written (their reservations came a level ago, so nobody waits for them),
+//    barrier, offsets (every wavefront scans the counts) and staging of level
+//    l.  1.2 M points of a late training iteration, 16 levels, 31 us of memory
+//    traffic at the copy rate: 569 -> 485 us, of which hashing, loads and
+//    products are 124, the group search and sums 128, ranks 82, staging 82,
+//    writes 68 (bound by the LDS and VALU instructions of 16 levels x 8
+//    corners; two workgroups of 8 wavefronts per CU, more gave nothing).
 //    Records beyond a list's capacity are added with fp32 atomics instead.
 //    The lists share one pool; bucket_layout_kernel (before the records)
 //    gives each list 5/4 of the records it took in the previous call on the
@@ -592,44 +599,35 @@ hash_bwd_lds_kernel(const float* __restrict__ x, int64_t n_cap, const int32_t* _
 //    a pool of at least 5/4 of a call's records holds every list of a call
 //    that repeats the previous one's counts: each list's share is then at
 //    least (5/4 c) * pool / (5/4 records + pool / 4) >= c.
-//    The largest |value| of each level is kept (integer max on the bits of a
-//    non-negative float: per wavefront by DPP, then one LDS atomic per
-//    wavefront and one global atomic per workgroup).
+//    A bound of each level's largest |value| is kept (integer max on the bits
+//    of a non-negative float: per wavefront by DPP, then one LDS atomic per
+//    wavefront and one global atomic per workgroup and level, on one of
+//    kMaxSlots words); at most 8 times the largest value.
 // 2. hash_bwd_bucket_sum_kernel: one workgroup per bucket sums its records in
 //    LDS as 64-bit fixed point (integer LDS atomics; scale 2^K with
-//    K = 61 - ceil(log2(count * max|value|)), so no sum can overflow and each
-//    record is rounded to count * max|value| * 2^-62 at worst, far below fp32
-//    resolution of anything but values ~2^-40 of the level's largest), then
+//    K = 61 - ceil(log2(count * bound)), so no sum can overflow and each
+//    record is rounded to count * max|value| * 2^-59 at worst, far below fp32
+//    resolution of anything but values ~2^-37 of the level's largest), then
 //    adds the sums to its rows, which no other workgroup touches.
 // Integer sums do not depend on the order, so the result is reproducible
 // (when no list overflows).
 constexpr int kBucketShift = 13;
 constexpr int kBucketEntries = 1 << kBucketShift;
+static_assert(2 * kBucketShift + 6 == 32, "two rows and one of 64 buckets in a word");
 constexpr int kMaxBucketsPerLevel = 512;
 // Same-cell lane groups of kMinGroup or more lanes are summed across lanes
-// (group_sums; measured on the late iterations of a full training run, ms
-// per hash-grid backward: a minimum of 3 / 4 / 5 / 6 / 8 lanes -> 1.07 /
-// 1.05 / 1.036 / 1.03 / 1.045: smaller groups cost more in cross-lane sums
-// than they save in records; with the cheaper ranks and staging of the
-// current record kernel 5 / 6 / 8 -> 0.897 / 0.901 / 0.901 ms, no difference); the search for groups (one leader per step,
-// lowest pending lane first) stops after kMaxSingles leaders in a row with a
-// smaller group (3 / 6 / 10 -> 1.05 / 1.03 / 1.044 ms), and is skipped on
-// levels where no lane shares the cell of the lane before it (the fine
-// levels).
-#ifndef SN_MIN_GROUP
-#define SN_MIN_GROUP 6
-#endif
-#ifndef SN_MAX_SINGLES
-#define SN_MAX_SINGLES 6
-#endif
-constexpr int kMinGroup = SN_MIN_GROUP;
-constexpr int kMaxSingles = SN_MAX_SINGLES;
-#ifndef SN_REC_THREADS
-#define SN_REC_THREADS 512
-#endif
-// points (lanes) per workgroup of the record kernel (the backward per late
-// launch of a full training run: 0.90 ms at 512, 1.22 ms at 256)
-constexpr int kRecThreads = SN_REC_THREADS;
+// (group_sums); the search for groups (one leader per step, lowest pending lane
+// first) stops after kMaxSingles leaders in a row with a smaller group, and is
+// skipped on levels where no lane shares the cell of the lane before it (the
+// fine levels).  1.2 M points, records + sums: kMinGroup / kMaxSingles 6 / 6
+// and 8 / 4 both 717 us (the latter has faster records and slower sums, as it
+// leaves more of them).
+constexpr int kMinGroup = 6;
+constexpr int kMaxSingles = 6;
+// Points (lanes) per workgroup of the record kernel: 256 makes half as long
+// runs per bucket and twice the reservations, 1024 leaves one workgroup per CU
+// to hide its barriers behind; both measured slower.
+constexpr int kRecThreads = 512;
 
 // Buckets of each level: level l owns global buckets [base[l], base[l+1]).
 struct BucketDesc {
@@ -639,7 +637,9 @@ struct BucketDesc {
 struct BucketPool {
   int32_t* hdr;       // [4] layout stamp: kLayoutMagic, n_buckets, total records
   int32_t* cursor;    // [n_buckets] records reserved per bucket (may exceed its cap)
-  uint32_t* maxbits;  // [kMaxLevels] bits of the largest |record value| per level
+  // [kMaxSlots][kMaxLevels] bits of the largest |record value| per level among
+  // the workgroups of a slot (a 128-byte line per slot)
+  uint32_t* maxbits;
   int32_t* start;     // [n_buckets] first pool index of each bucket's list
   int32_t* bcap;      // [n_buckets] list capacity
   uint16_t* row;      // [total] row within the bucket
@@ -648,6 +648,12 @@ struct BucketPool {
 };
 
 constexpr int32_t kLayoutMagic = 0x4c594f54;
+// Workgroup b of the record kernel keeps its levels' maxima in slot b %
+// kMaxSlots: global atomics on one word are served one after another (~9 ns
+// each, measured), and one word per level for the 2352 workgroups of a 1.2
+// M-point launch holds the kernel up: 531 us, 485 with slots (without the group
+// search 436 and 124).
+constexpr int kMaxSlots = 64;
 // Largest list unless the pool's even split is larger: the sum kernel takes
 // a list in one workgroup, whose integer LDS atomics (~5e9 lane ops/s per CU)
 // make a list of n records last at least n * F / 5e9 s; records beyond it
@@ -717,6 +723,7 @@ bucket_layout_kernel(BucketPool pool, int32_t nb) {
   for (int q = 0; q < kPer; ++q) {
     if (scale) want[q] = (int64_t)(((uint64_t)want[q] * factor) >> 32);
     else want[q] = want[q] > 0 ? min(want[q] + extra, cap) : 0;  // want <= cap already
+    want[q] &= ~(int64_t)1;  // whole pairs of records; every start is even
     mine += want[q];
   }
   // exclusive scan of the per-thread sums
@@ -739,7 +746,7 @@ bucket_layout_kernel(BucketPool pool, int32_t nb) {
       run += want[q];
     }
   }
-  if (tid < kMaxLevels) pool.maxbits[tid] = 0u;
+  for (int k = tid; k < kMaxSlots * kMaxLevels; k += kLayoutThreads) pool.maxbits[k] = 0u;
   if (tid == 0) {
     pool.hdr[0] = kLayoutMagic;
     pool.hdr[1] = nb;
@@ -799,13 +806,12 @@ __device__ __forceinline__ void group_sums(float (&a)[8 * F], int lane, int ld, 
   }
 }
 
-// Records of one level wait in LDS, ordered by bucket, before they are
-// written: a bucket's records from one workgroup are consecutive in its list,
-// so the writes of consecutive staging entries are consecutive in memory.
-struct StagedRecord {
-  uint32_t key;  // row within the level
-  int32_t rank;  // position among the workgroup's records of its bucket
-  float v[2];
+// Records of one level wait in LDS as x pairs, ordered by bucket, before they
+// are written: a bucket's pairs from one workgroup are consecutive in its
+// list, so the writes of consecutive staging entries are consecutive in memory.
+template <int F>
+struct alignas(8 * F) PairValues {
+  float v[2 * F];  // values of the pair's two rows
 };
 
 // kAd: the records also carry the table's part of the double backward
@@ -813,7 +819,9 @@ struct StagedRecord {
 // fp32 atomics): with the x-gradient's cotangent v = gv[i] and the cotangent
 // genc2 of the encoding's derivative along v, corner c of level l adds
 // scale_l (v . d w_c / d frac) genc2[i, l, f] to row idx_c, feature f.
-template <int F, bool kAd = false>
+// kMaxPer: buckets per lane of the scan (1, 4, 8: levels of at most 64, 256,
+// 512 buckets, T <= 2^19, 2^21, 2^22; its reservations live in registers).
+template <int F, bool kAd, int kMaxPer>
 __global__ void __launch_bounds__(kRecThreads, 4)  // 4 wavefronts per SIMD: 2 workgroups per CU
 hash_bwd_rec_kernel(const float* __restrict__ x, int64_t n_cap, const int32_t* __restrict__ n_dev,
                     const float* __restrict__ params, HashGridDesc d,
@@ -821,20 +829,30 @@ hash_bwd_rec_kernel(const float* __restrict__ x, int64_t n_cap, const int32_t* _
                     float* __restrict__ gx, BucketDesc bd, BucketPool pool,
                     const float* __restrict__ gv = nullptr,
                     const float* __restrict__ genc2 = nullptr) {
-  __shared__ int32_t hist[kMaxBucketsPerLevel];   // records per bucket (this level)
-  __shared__ int32_t lofs[kMaxBucketsPerLevel];   // their first staging slot
-  // per bucket: (list room left at the workgroup's share, pool index of the
-  // share's first record)
-  __shared__ int2 rres[kMaxBucketsPerLevel];
-  __shared__ StagedRecord stage[kRecThreads * 8];
-  __shared__ uint32_t lmax;
-  __shared__ int32_t n_staged;
+  // what one pass (a level, or a level's split pairs) hands to the next is
+  // double-buffered by the pass number's parity
+  constexpr int kBuckets = 64 * kMaxPer;
+  __shared__ int32_t hist[2][kBuckets];  // pairs per bucket
+  __shared__ int32_t lofs[kBuckets];     // a bucket's first staging slot
+  // per bucket: twice the first staging slot past the list's room, and the
+  // pool index of staging slot 0 seen from this bucket's list (so that the
+  // pair in slot q belongs at pool index y + 2q while 2q < x)
+  __shared__ int2 rres[kBuckets];
+  __shared__ PairValues<F> stage_v[kRecThreads * 4];
+  // the pair's rows within the bucket (13 bits each) and, above them, its
+  // bucket; more than 64 buckets per level: the bucket in a word of its own
+  __shared__ uint32_t stage_r[kRecThreads * 4];
+  __shared__ uint16_t stage_b[kMaxPer == 1 ? 1 : kRecThreads * 4];
+  __shared__ uint32_t lmax[2];
+  __shared__ int32_t split[2];  // whether some pair of the pass lies in two buckets
   const int tid = threadIdx.x, lane = tid & 63;
-  for (int b = tid; b < kMaxBucketsPerLevel; b += kRecThreads) hist[b] = 0;
-  if (tid == 0) lmax = 0u;
+  const bool wave0 = __builtin_amdgcn_readfirstlane(tid >> 6) == 0;
+  for (int b = tid; b < 2 * kBuckets; b += kRecThreads) (&hist[0][0])[b] = 0;
+  if (tid < 2) lmax[tid] = 0u, split[tid] = 0;
   __syncthreads();
   const int64_t n = dev_count(n_cap, n_dev);
   const int64_t n_chunks = ceil_div(n, kRecThreads);
+  int par = 0;
   for (int64_t ch = blockIdx.x; ch < n_chunks; ch += gridDim.x) {  // uniform per workgroup
     const int64_t i = ch * kRecThreads + tid;
     const bool act = i < n;
@@ -857,6 +875,50 @@ hash_bwd_rec_kernel(const float* __restrict__ x, int64_t n_cap, const int32_t* _
     const bool vec_g = F == 2 && (d.n_levels & 3) == 0 &&
                        (reinterpret_cast<uintptr_t>(genc) & 15) == 0;
     float4 gq0 = make_float4(0.f, 0.f, 0.f, 0.f), gq1 = gq0;
+    // the previous pass, whose pairs are staged but not written yet: their
+    // number, the level's rows, and (wavefront 0) its lists' reservations
+    int prev_n = 0, prev_nb = 0;
+    float* prev_tg = nullptr;
+    // (count, position in the list, the list's capacity and start, staging slot)
+    int32_t res_c[kMaxPer], res_r0[kMaxPer], res_cap[kMaxPer], res_st[kMaxPer], res_l[kMaxPer];
+    // wavefront 0: the reservations of the previous pass as (limit, base)
+    auto publish = [&]() {
+      const int per = kMaxPer == 1 ? 1 : (prev_nb + 63) / 64;
+#pragma unroll
+      for (int q = 0; q < kMaxPer; ++q) {
+        const int b = lane * per + q;
+        if (q < per && b < prev_nb && res_c[q]) {
+          // (even counts, capacities and starts: a pair is inside or outside)
+          rres[b] = make_int2(2 * res_l[q] + (res_cap[q] - res_r0[q]),
+                              res_st[q] + res_r0[q] - 2 * res_l[q]);
+        }
+      }
+    };
+    // the previous pass's pairs from LDS to their lists (beyond a list's
+    // room: fp32 atomics)
+    auto write_out = [&]() {
+      for (int q = tid; q < prev_n; q += kRecThreads) {
+        const uint32_t key = stage_r[q];
+        const uint32_t b = kMaxPer == 1 ? key >> (2 * kBucketShift) : stage_b[q];
+        const uint32_t row0 = key & (kBucketEntries - 1);
+        const uint32_t row1 = (key >> kBucketShift) & (kBucketEntries - 1);
+        const PairValues<F> e = stage_v[q];
+        const int2 rr = rres[b];
+        if (2 * q < rr.x) {
+          const int64_t at = rr.y + 2 * (int64_t)q;
+          reinterpret_cast<uint32_t*>(pool.row)[at >> 1] = row0 | (row1 << 16);
+          *reinterpret_cast<PairValues<F>*>(pool.val + at * F) = e;
+        } else {
+          float* t0 = prev_tg + ((int64_t)b * kBucketEntries + row0) * F;
+          float* t1 = prev_tg + ((int64_t)b * kBucketEntries + row1) * F;
+#pragma unroll
+          for (int f = 0; f < F; ++f) {
+            atomicAdd(&t0[f], e.v[f]);
+            if (e.v[F + f] != 0.f) atomicAdd(&t1[f], e.v[F + f]);
+          }
+        }
+      }
+    };
     for (int l = 0, na_ = active_levels(d); l < na_; ++l) {
       float gl[F];
       if (vec_g) {
@@ -898,7 +960,23 @@ hash_bwd_rec_kernel(const float* __restrict__ x, int64_t n_cap, const int32_t* _
           for (int f = 0; f < F; ++f) rv[c][f] += a * g2[f];
         }
       }
-      bool has = act;
+      if (gx && act) {
+        float dw[8][3];
+        hg_dweights(fr, dw);
+        const float* tab = params + (int64_t)d.offset[l] * F;
+        float acc[3] = {0.f, 0.f, 0.f};
+#pragma unroll
+        for (int c = 0; c < 8; ++c) {
+          float sm = 0.f;
+#pragma unroll
+          for (int f = 0; f < F; ++f) sm += gl[f] * tab[(int64_t)idx[c] * F + f];
+#pragma unroll
+          for (int k = 0; k < 3; ++k) acc[k] += dw[c][k] * sm;
+        }
+#pragma unroll
+        for (int k = 0; k < 3; ++k) dx[k] += d.scale[l] * acc[k];
+      }
+      bool has = act, lead = false;
       uint64_t pend = __ballot(act);
       {
         // the previous lane's cell by a DPP wave shift (wave_shr:1), not an
@@ -925,28 +1003,30 @@ hash_bwd_rec_kernel(const float* __restrict__ x, int64_t n_cap, const int32_t* _
             for (int f = 0; f < F; ++f) a[c * F + f] = in ? rv[c][f] : 0.f;
           group_sums<F>(a, lane, ld, rv);
           if (in && lane != ld) has = false;
+          lead = lead || lane == ld;
           singles = 0;
         } else if (++singles >= kMaxSingles) {
           break;
         }
         pend &= ~m;
       }
-      // ranks within the workgroup's share of each bucket
-      const int gb0 = bd.base[l], nb = bd.base[l + 1] - gb0;
-      int32_t rank[8];
-      // largest |value| as bits: the bits of |x| order like |x| for finite
-      // values and inf, and every NaN's bits are above inf's, so a NaN or inf
-      // reaches the level maximum and the sums fall back to fp32 (fmaxf would
-      // drop a NaN)
+      // a bound of the lane's largest |value| as bits: |dL/denc| of an unmerged
+      // lane (its weights are at most 1 and the largest at least 1/8; NaN at a
+      // position that is not finite), the sums of a merged one.  The bits of |x| order like |x| for finite values and
+      // inf, and every NaN's bits are above inf's, so a NaN or inf reaches the
+      // level maximum and the sums fall back to fp32 (fmaxf would drop a NaN)
       uint32_t vmaxb = 0u;
-      if (has) {
+      if (!kAd && !lead) {
 #pragma unroll
-        for (int c = 0; c < 8; ++c) {
-          rank[c] = atomicAdd(&hist[idx[c] >> kBucketShift], 1);
+        for (int f = 0; f < F; ++f) vmaxb = max(vmaxb, __float_as_uint(fabsf(gl[f])));
+        if (!(fr[0] + fr[1] + fr[2] <= 3.f)) vmaxb = 0x7fc00000u;
+      } else {
+#pragma unroll
+        for (int c = 0; c < 8; ++c)
 #pragma unroll
           for (int f = 0; f < F; ++f) vmaxb = max(vmaxb, __float_as_uint(fabsf(rv[c][f])));
-        }
       }
+      if (!has) vmaxb = 0u;
       // the wavefront's maximum (prefix maxima within rows, then across rows:
       // lane 63 ends with it), one LDS atomic per wavefront instead of one
       // per lane on the same word (record kernel 592 -> 536 us per late launch)
@@ -956,139 +1036,122 @@ hash_bwd_rec_kernel(const float* __restrict__ x, int64_t n_cap, const int32_t* _
       vmaxb = max(vmaxb, dpp_u<0x118>(vmaxb));
       vmaxb = max(vmaxb, dpp_u<0x142, 0xa>(vmaxb));
       vmaxb = max(vmaxb, dpp_u<0x143, 0xc>(vmaxb));
-      if (lane == 63 && vmaxb) atomicMax(&lmax, vmaxb);
-      if (gx && act) {
-        float dw[8][3];
-        hg_dweights(fr, dw);
-        const float* tab = params + (int64_t)d.offset[l] * F;
-        float acc[3] = {0.f, 0.f, 0.f};
+      if (lane == 63 && vmaxb) atomicMax(&lmax[par], vmaxb);
+      const int gb0 = bd.base[l], nb = bd.base[l + 1] - gb0;
+      const int per = kMaxPer == 1 ? 1 : (nb + 63) / 64;  // buckets per lane of the scan, in order
+      // One pass takes the level's x pairs; a pair whose rows lie in two
+      // buckets (a dense level's bucket boundary, a hashed level's x cell -1)
+      // leaves its first row there, beside an empty one, and its second row in
+      // a second pass that only such levels have.
+      auto pass = [&](auto second_c) {
+        constexpr bool second = decltype(second_c)::value;
+        int32_t rank[4];
+        bool emit[4];
 #pragma unroll
-        for (int c = 0; c < 8; ++c) {
-          float sm = 0.f;
-#pragma unroll
-          for (int f = 0; f < F; ++f) sm += gl[f] * tab[(int64_t)idx[c] * F + f];
-#pragma unroll
-          for (int k = 0; k < 3; ++k) acc[k] += dw[c][k] * sm;
-        }
-#pragma unroll
-        for (int k = 0; k < 3; ++k) dx[k] += d.scale[l] * acc[k];
-      }
-      __syncthreads();
-      // wavefront 0 alone: staging offsets (exclusive scan of the counts);
-      // with one bucket per lane (nb <= 64) it first issues the lane's list
-      // reservation (one global atomic per non-empty bucket: position
-      // relative to the list), whose result it needs only after the scan,
-      // the barrier below and its own staging: the barrier waits for LDS
-      // operations only, so the round trip overlaps all three
-      int32_t res_c = 0, res_r0 = 0;
-      if (tid < 64) {
-        const int per = (nb + 63) / 64;  // buckets per lane, in order
-        int sum = 0;
-        for (int q = 0; q < per; ++q) {
-          const int b = tid * per + q;
-          if (b < nb) sum += hist[b];
-        }
-        if (nb <= 64) {
-          res_c = sum;
-          if (res_c) res_r0 = atomicAdd(&pool.cursor[gb0 + tid], res_c);
-        }
-        // inclusive scan across the wavefront on DPP lane moves (row shifts,
-        // then the rows' totals broadcast upwards), no LDS round trips
-        uint32_t incl = (uint32_t)sum;
-        incl += dpp_u<0x111>(incl);
-        incl += dpp_u<0x112>(incl);
-        incl += dpp_u<0x114>(incl);
-        incl += dpp_u<0x118>(incl);
-        incl += dpp_u<0x142, 0xa>(incl);
-        incl += dpp_u<0x143, 0xc>(incl);
-        int run = (int)incl - sum;
-        for (int q = 0; q < per; ++q) {
-          const int b = tid * per + q;
-          if (b < nb) {
-            lofs[b] = run;
-            run += hist[b];
+        for (int q = 0; q < 4; ++q) {
+          const uint32_t b0 = idx[2 * q] >> kBucketShift, b1 = idx[2 * q + 1] >> kBucketShift;
+          emit[q] = has && (!second || b0 != b1);
+          if (emit[q]) {
+            rank[q] = atomicAdd(&hist[par][second ? b1 : b0], 1);
+            if (!second && b0 != b1) split[par] = 1;
           }
         }
-        if (tid == 63) n_staged = (int)incl;
-      }
-      if (tid == 0) {
-        atomicMax(&pool.maxbits[l], lmax);
-        lmax = 0u;
-      }
-      __syncthreads();
-      // every wavefront stages its records (the staging needs only the
-      // offsets); wavefront 0 then turns the reservations into (room, pool
-      // index while in room) per bucket -- with several buckets per lane it
-      // takes them here -- and sets the counts back to zero
-      auto stage_own = [&]() {
-        if (has) {
+        if (wave0) publish();
+        __syncthreads();
+        // wavefront 0: room for this pass's pairs in the lists, one global
+        // atomic per non-empty bucket; the results are needed in the next pass
+        if (wave0) {
 #pragma unroll
-          for (int c = 0; c < 8; ++c) {
-            StagedRecord& e = stage[lofs[idx[c] >> kBucketShift] + rank[c]];
-            e.key = idx[c];
-            e.rank = rank[c];
+          for (int q = 0; q < kMaxPer; ++q) {
+            const int b = lane * per + q;
+            res_c[q] = q < per && b < nb ? hist[par][b] : 0;
+          }
 #pragma unroll
-            for (int f = 0; f < F; ++f) e.v[f] = rv[c][f];
-          }
-        }
-      };
-      if (tid < 64) {
-        if (nb <= 64) {
-          stage_own();
-          if (res_c) {
-            const int32_t room = pool.bcap[gb0 + tid] - res_r0;
-            rres[tid] = make_int2(room, room > 0 ? pool.start[gb0 + tid] + res_r0 : 0);
-          }
-          if (tid < nb) hist[tid] = 0;
-        } else {
-          stage_own();
-          const int per = (nb + 63) / 64;
-          for (int q = 0; q < per; ++q) {
-            const int b = tid * per + q;
-            if (b < nb) {
-              const int32_t c = hist[b];
-              if (c) {
-                const int32_t r0 = atomicAdd(&pool.cursor[gb0 + b], c);
-                const int32_t room = pool.bcap[gb0 + b] - r0;
-                rres[b] = make_int2(room, room > 0 ? pool.start[gb0 + b] + r0 : 0);
-              }
-              hist[b] = 0;
+          for (int q = 0; q < kMaxPer; ++q)
+            if (res_c[q]) {
+              const int gb = gb0 + lane * per + q;
+              res_r0[q] = atomicAdd(&pool.cursor[gb], 2 * res_c[q]);
+              res_cap[q] = pool.bcap[gb];
+              res_st[q] = pool.start[gb];
             }
-          }
         }
-      } else {
-        stage_own();
-      }
-      __syncthreads();
-      {
-        float* tg = gparams + (int64_t)d.offset[l] * F;
-        const int ns = n_staged;
-        auto put = [&](const StagedRecord& e, int2 rr) {
-          if (e.rank < rr.x) {
-            const int64_t at = rr.y + e.rank;
-            pool.row[at] = (uint16_t)(e.key & (kBucketEntries - 1));
+        const bool again = !second && split[par];  // uniform
+        if (tid == 64) {
+          if (lmax[par])
+            atomicMax(&pool.maxbits[(blockIdx.x % kMaxSlots) * kMaxLevels + l], lmax[par]);
+          lmax[par] = 0u;
+        }
+        // the other buffer's counts were last read before the barrier above
+        for (int b = tid; b < kBuckets; b += kRecThreads) hist[par ^ 1][b] = 0;
+        if (tid == 128) split[par ^ 1] = 0;
+        write_out();
+        __syncthreads();
+        // staging offsets: every wavefront scans the counts (inclusive scan on
+        // DPP lane moves: row shifts, then the rows' totals broadcast upwards)
+        {
+          int cnt[kMaxPer], sum = 0;
 #pragma unroll
-            for (int f = 0; f < F; ++f) pool.val[at * F + f] = e.v[f];
+          for (int q = 0; q < kMaxPer; ++q) {
+            const int b = lane * per + q;
+            cnt[q] = q < per && b < nb ? hist[par][b] : 0;
+            sum += cnt[q];
+          }
+          uint32_t incl = (uint32_t)sum;
+          incl += dpp_u<0x111>(incl);
+          incl += dpp_u<0x112>(incl);
+          incl += dpp_u<0x114>(incl);
+          incl += dpp_u<0x118>(incl);
+          incl += dpp_u<0x142, 0xa>(incl);
+          incl += dpp_u<0x143, 0xc>(incl);
+          int run = (int)incl - sum;
+          // every wavefront writes the same values; it reads only after its own
+#pragma unroll
+          for (int q = 0; q < kMaxPer; ++q) {
+            const int b = lane * per + q;
+            if (q < per && b < nb) lofs[b] = run;
+            res_l[q] = run;
+            run += cnt[q];
+          }
+          prev_n = __builtin_amdgcn_readlane((int)incl, 63);
+          __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        }
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          if (!emit[q]) continue;
+          const uint32_t i0 = idx[2 * q], i1 = idx[2 * q + 1];
+          const uint32_t b0 = i0 >> kBucketShift, b1 = i1 >> kBucketShift;
+          const uint32_t b = second ? b1 : b0;
+          const bool both = b0 == b1;
+          const int at = lofs[b] + rank[q];
+          const uint32_t r0 = (second ? i1 : i0) & (kBucketEntries - 1);
+          const uint32_t r1 = both ? i1 & (kBucketEntries - 1) : r0;
+          PairValues<F> e;
+#pragma unroll
+          for (int f = 0; f < F; ++f) {
+            e.v[f] = second ? rv[2 * q + 1][f] : rv[2 * q][f];
+            e.v[F + f] = both ? rv[2 * q + 1][f] : 0.f;
+          }
+          stage_v[at] = e;
+          const uint32_t key = r0 | (r1 << kBucketShift);
+          if constexpr (kMaxPer == 1) {
+            stage_r[at] = key | (b << (2 * kBucketShift));  // b < 64
           } else {
-#pragma unroll
-            for (int f = 0; f < F; ++f) atomicAdd(&tg[(int64_t)e.key * F + f], e.v[f]);
+            stage_r[at] = key;
+            stage_b[at] = (uint16_t)b;
           }
-        };
-        // two records per lane and step, both read from LDS before either is
-        // written out (record kernel 527 -> 516 us per late launch)
-        int q = tid;
-        for (; q + kRecThreads < ns; q += 2 * kRecThreads) {
-          const StagedRecord e0 = stage[q], e1 = stage[q + kRecThreads];
-          const int2 r0 = rres[e0.key >> kBucketShift], r1 = rres[e1.key >> kBucketShift];
-          put(e0, r0);
-          put(e1, r1);
         }
-        if (q < ns) {
-          const StagedRecord e = stage[q];
-          put(e, rres[e.key >> kBucketShift]);
-        }
-      }
+        prev_nb = nb;
+        prev_tg = gparams + (int64_t)d.offset[l] * F;
+        par ^= 1;
+        return again;
+      };
+      if (pass(std::false_type{})) pass(std::true_type{});
     }
+    // the last pass's pairs
+    if (wave0) publish();
+    __syncthreads();
+    write_out();
+    if (ch + gridDim.x < n_chunks) __syncthreads();  // uniform: the next chunk stages again
     if (gx && act) {
 #pragma unroll
       for (int k = 0; k < 3; ++k) gx[3 * i + k] = dx[k];
@@ -1096,35 +1159,24 @@ hash_bwd_rec_kernel(const float* __restrict__ x, int64_t n_cap, const int32_t* _
   }
 }
 
-// round(v * 2^K) as a 64-bit integer (round half to even, the result of
-// llrint on the exact product), from the bits of v: v = m * 2^(e - 150), so
-// v * 2^K = m * 2^(e - 150 + K), a shift of the 24-bit significand.  The
-// caller guarantees |v| * 2^K < 2^62 and finite v.  Integer ops only.
-__device__ __forceinline__ long long fixed_of(float v, int K) {
-  const uint32_t b = __float_as_uint(v);
-  const int e = (int)((b >> 23) & 0xffu);
-  uint32_t m = b & 0x7fffffu;
-  int sh;
-  if (e) {
-    m |= 0x800000u;
-    sh = e - 150 + K;
-  } else {
-    sh = -149 + K;  // subnormal: m * 2^-149
-  }
-  unsigned long long q;
-  if (sh >= 0) {
-    q = (unsigned long long)m << sh;
-  } else if (sh < -25) {
-    q = 0ull;  // below half of the last unit
-  } else {
-    const int r = -sh;
-    const uint32_t half = 1u << (r - 1);
-    const uint32_t rem = m & ((1u << r) - 1u);
-    uint32_t t = m >> r;
-    if (rem > half || (rem == half && (t & 1u))) ++t;
-    q = t;
-  }
-  return (b >> 31) ? -(long long)q : (long long)q;
+// round(v * 2^K) as a 64-bit integer (round half to even: the result of
+// llrint on the exact product), |v| * 2^K < 2^62 and v finite: |v| * 2^(K-32)
+// split into its whole part (the high word) and the rest, which is exact in
+// fp32 and gives the low word.  The power of two is applied in two halves sh =
+// 2^h1, sl = 2^h2 (h1 + h2 = K - 32), each a normal fp32 number; a value so
+// small that the product is subnormal is below half of the last unit.  Integer
+// and fp32 operations only (12 against ~30 of a shift of the significand with
+// its cases: with the paired loads the sum kernel went from 262 to 230 us for the
+// 1.2 M points of a late training iteration).
+__device__ __forceinline__ unsigned long long fixed_of(float v, float sh, float sl) {
+  const float a = (fabsf(v) * sh) * sl;
+  const uint32_t hi = (uint32_t)a;
+  const float rest = (a - (float)hi) * 4294967296.f;
+  // (rest < 2^32: fp32 has no value between 2^32 - 256 and 2^32)
+  const uint32_t lo = (uint32_t)__builtin_rintf(rest);
+  const unsigned long long q = ((unsigned long long)hi << 32) | lo;
+  const unsigned long long sgn = (unsigned long long)((long long)(int)__float_as_uint(v) >> 63);
+  return (q ^ sgn) - sgn;
 }
 
 // 2^e with count * vmax < 2^e (e from the fp32 product; rounding can only
@@ -1144,7 +1196,16 @@ hash_bwd_bucket_sum_kernel(HashGridDesc d, BucketDesc bd, BucketPool pool,
   int l = 0;
   while (l + 1 < d.n_levels && bd.base[l + 1] <= gb) ++l;
   const int32_t nrec = min(pool.cursor[gb], pool.bcap[gb]);
-  const float vmax = __uint_as_float(pool.maxbits[l]);
+  // the level's largest |value| over the slots (every wavefront for itself)
+  static_assert(kMaxSlots == 64, "one slot per lane");
+  uint32_t vb = pool.maxbits[(tid & 63) * kMaxLevels + l];
+  vb = max(vb, dpp_u<0x111>(vb));
+  vb = max(vb, dpp_u<0x112>(vb));
+  vb = max(vb, dpp_u<0x114>(vb));
+  vb = max(vb, dpp_u<0x118>(vb));
+  vb = max(vb, dpp_u<0x142, 0xa>(vb));
+  vb = max(vb, dpp_u<0x143, 0xc>(vb));
+  const float vmax = __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)vb, 63));
   if (nrec <= 0 || vmax == 0.f) return;  // uniform per workgroup
   const int64_t at0 = pool.start[gb];
   const int64_t e0 = (int64_t)(gb - bd.base[l]) * kBucketEntries;
@@ -1165,38 +1226,38 @@ hash_bwd_bucket_sum_kernel(HashGridDesc d, BucketDesc bd, BucketPool pool,
     return;
   }
   const int K = 61 - bound_exp(vmax, nrec);  // count * max|value| < 2^(61 - K)
+  // 2^(K - 32) as two normal factors (-98 <= K <= 210)
+  const int h1 = (K - 32) / 2, h2 = K - 32 - h1;
+  const float sh = ldexpf(1.f, h1), sl = ldexpf(1.f, h2);
   for (int j = tid; j < kBucketEntries * F; j += 1024) acc[j] = 0ull;
   __syncthreads();
-  // kU records per lane in flight: their loads are issued before the first
-  // LDS atomic (one workgroup per CU, so the loads' latency is hidden here;
-  // 8 against 4: 254 -> 251.5 us per late launch, the LDS atomics being the
-  // rest of it)
-#ifndef SN_SUM_UNROLL
-#define SN_SUM_UNROLL 8
-#endif
-  constexpr int kU = SN_SUM_UNROLL;
+  // kU pairs of records per lane in flight: their loads (4 + 8 F bytes each)
+  // are issued before the first LDS atomic (one workgroup per CU, so the
+  // loads' latency is hidden here)
+  constexpr int kU = 4;
+  const uint32_t* rows2 = reinterpret_cast<const uint32_t*>(pool.row) + (at0 >> 1);
+  const PairValues<F>* vals2 = reinterpret_cast<const PairValues<F>*>(pool.val + at0 * F);
+  auto add = [&](uint32_t rr, const PairValues<F>& e) {
+#pragma unroll
+    for (int f = 0; f < F; ++f) {
+      atomicAdd(&acc[(rr & 0xffffu) * F + f], fixed_of(e.v[f], sh, sl));
+      atomicAdd(&acc[(rr >> 16) * F + f], fixed_of(e.v[F + f], sh, sl));
+    }
+  };
+  const int32_t np = nrec >> 1;
   int r = tid;
-  for (; r + (kU - 1) * 1024 < nrec; r += kU * 1024) {
-    int row[kU];
-    float v[kU][F];
+  for (; r + (kU - 1) * 1024 < np; r += kU * 1024) {
+    uint32_t row[kU];
+    PairValues<F> e[kU];
 #pragma unroll
     for (int u = 0; u < kU; ++u) {
-      row[u] = pool.row[at0 + r + u * 1024];
-#pragma unroll
-      for (int f = 0; f < F; ++f) v[u][f] = pool.val[(at0 + r + u * 1024) * F + f];
+      row[u] = rows2[r + u * 1024];
+      e[u] = vals2[r + u * 1024];
     }
 #pragma unroll
-    for (int u = 0; u < kU; ++u)
-#pragma unroll
-      for (int f = 0; f < F; ++f)
-        atomicAdd(&acc[row[u] * F + f], (unsigned long long)fixed_of(v[u][f], K));
+    for (int u = 0; u < kU; ++u) add(row[u], e[u]);
   }
-  for (; r < nrec; r += 1024) {
-    const int row = pool.row[at0 + r];
-#pragma unroll
-    for (int f = 0; f < F; ++f)
-      atomicAdd(&acc[row * F + f], (unsigned long long)fixed_of(pool.val[(at0 + r) * F + f], K));
-  }
+  for (; r < np; r += 1024) add(rows2[r], vals2[r]);
   __syncthreads();
   // sum * 2^-K: the int64 -> fp32 conversion rounds once, the scaling is exact
   for (int64_t j = tid; j < rows * F; j += 1024) {
@@ -1219,10 +1280,13 @@ static int64_t make_bucket_desc(const HashGridDesc& d, BucketDesc* bd) {
   return tot;
 }
 
-// workspace: hdr[4] | cursor[nb] | maxbits[kMaxLevels] | start[nb] | bcap[nb] |
-//            row[total] | val[total*F]
-static size_t bucket_head_bytes(int64_t n_buckets) {
+// workspace: hdr[4] | cursor[nb] | (kMaxLevels words unused) | start[nb] |
+//            bcap[nb] | maxbits[kMaxSlots][kMaxLevels] | row[total] | val[total*F]
+static size_t bucket_list_bytes(int64_t n_buckets) {
   return align_up(sizeof(int32_t) * (4 + 3 * n_buckets + kMaxLevels), 256);
+}
+static size_t bucket_head_bytes(int64_t n_buckets) {
+  return bucket_list_bytes(n_buckets) + sizeof(uint32_t) * kMaxSlots * kMaxLevels;
 }
 static size_t bucket_ws_bytes(int64_t n_buckets, int F, int64_t total) {
   return bucket_head_bytes(n_buckets) + align_up(sizeof(uint16_t) * total, 256) +
@@ -1482,6 +1546,11 @@ static int hashgrid_bwd_impl(const float* x, int64_t n_cap, const int32_t* n_dev
     const int64_t nb = make_bucket_desc(d, &bd);
     const bool buckets = workspace && nb > 0 && n_cap < (1ll << 28) - 4096 && d.n_active > 0;
     if (buckets) {
+      // pairs are read and written 16 bytes at a time
+      char* w = static_cast<char*>(workspace);
+      const size_t skip = (16 - (reinterpret_cast<uintptr_t>(w) & 15)) & 15;
+      w += skip;
+      workspace_bytes = workspace_bytes > skip ? workspace_bytes - skip : 0;
       const size_t head = bucket_head_bytes(nb);
       const size_t per = sizeof(uint16_t) + sizeof(float) * n_features;
       int64_t total =
@@ -1493,11 +1562,10 @@ static int hashgrid_bwd_impl(const float* x, int64_t n_cap, const int32_t* n_dev
                   workspace_bytes);
         return SN_ESPACE;
       }
-      char* w = static_cast<char*>(workspace);
       BucketPool pool;
       pool.hdr = reinterpret_cast<int32_t*>(w);
       pool.cursor = pool.hdr + 4;
-      pool.maxbits = reinterpret_cast<uint32_t*>(pool.cursor + nb);
+      pool.maxbits = reinterpret_cast<uint32_t*>(w + bucket_list_bytes(nb));
       pool.start = pool.cursor + nb + kMaxLevels;
       pool.bcap = pool.start + nb;
       pool.row = reinterpret_cast<uint16_t*>(w + head);
@@ -1509,20 +1577,25 @@ static int hashgrid_bwd_impl(const float* x, int64_t n_cap, const int32_t* n_dev
       if (rc) return rc;
       const unsigned rgrid = grid_for(n_cap, kRecThreads, kHashBlocks);
       const bool ad = gv && genc2;
-      if (n_features == 1 && ad)
-        hash_bwd_rec_kernel<1, true><<<rgrid, kRecThreads, 0, s>>>(
-            x, n_cap, n_dev, params, d, grad_enc, grad_params, grad_x, bd, pool, gv, genc2);
-      else if (n_features == 1)
-        hash_bwd_rec_kernel<1><<<rgrid, kRecThreads, 0, s>>>(x, n_cap, n_dev, params, d,
-                                                             grad_enc, grad_params, grad_x, bd,
-                                                             pool);
-      else if (ad)
-        hash_bwd_rec_kernel<2, true><<<rgrid, kRecThreads, 0, s>>>(
-            x, n_cap, n_dev, params, d, grad_enc, grad_params, grad_x, bd, pool, gv, genc2);
-      else
-        hash_bwd_rec_kernel<2><<<rgrid, kRecThreads, 0, s>>>(x, n_cap, n_dev, params, d,
-                                                             grad_enc, grad_params, grad_x, bd,
-                                                             pool);
+      int max_nb = 0;
+      for (int l = 0; l < d.n_active; ++l) max_nb = std::max(max_nb, bd.base[l + 1] - bd.base[l]);
+#define SN_REC(F_, AD_)                                                                       \
+  do {                                                                                        \
+    if (max_nb <= 64)                                                                         \
+      hash_bwd_rec_kernel<F_, AD_, 1><<<rgrid, kRecThreads, 0, s>>>(                          \
+          x, n_cap, n_dev, params, d, grad_enc, grad_params, grad_x, bd, pool, gv, genc2);    \
+    else if (max_nb <= 256)                                                                   \
+      hash_bwd_rec_kernel<F_, AD_, 4><<<rgrid, kRecThreads, 0, s>>>(                          \
+          x, n_cap, n_dev, params, d, grad_enc, grad_params, grad_x, bd, pool, gv, genc2);    \
+    else                                                                                      \
+      hash_bwd_rec_kernel<F_, AD_, kMaxBucketsPerLevel / 64><<<rgrid, kRecThreads, 0, s>>>(   \
+          x, n_cap, n_dev, params, d, grad_enc, grad_params, grad_x, bd, pool, gv, genc2);    \
+  } while (0)
+      if (n_features == 1 && ad) SN_REC(1, true);
+      else if (n_features == 1) SN_REC(1, false);
+      else if (ad) SN_REC(2, true);
+      else SN_REC(2, false);
+#undef SN_REC
       *bucketed = ad ? 1 : 0;
       rc = check_launch("sn_hashgrid_bwd");
       if (rc) return rc;
