@@ -334,6 +334,30 @@ int sn_mlp_bwd_ad_enc(const float* x, const float* enc, const float* v, const fl
                       float* g_enc, float* g_enc_dot, float* g_mlp, int32_t accumulate,
                       void* workspace, size_t workspace_bytes, void* stream);
 
+/* The encoding by levels: enc [n_levels, n_cap, 2] (two features per level), */
+/* the values of sn_hashgrid_fwd_dev / _fwd16_dev (params16 when given); and  */
+/* the MLP on it (enc_dims = 2 n_levels, a multiple of 4; enc and g_enc       */
+/* 16-byte aligned; g_enc stays [n, enc_dims]).                               */
+int sn_hashgrid_fwd_levels_dev(const float* x, int64_t n_cap, const int32_t* n_dev,
+                               const float* params, const void* params16, int32_t n_levels,
+                               int32_t log2_hashmap_size, int32_t base_resolution,
+                               float per_level_scale, int32_t n_active_levels,
+                               const int32_t* n_active_dev, float* enc, void* stream);
+int sn_mlp_fwd_levels(const float* x, const float* enc, int32_t enc_dims, int64_t n_cap,
+                      const int32_t* n_dev, const float* mlp, int32_t d_hidden, int32_t n_layers,
+                      float beta, float* sdf, float* dsdf_dh0, void* stream);
+int sn_mlp_bwd_levels(const float* x, const float* enc, int32_t enc_dims, int64_t n_cap,
+                      const int32_t* n_dev, const float* mlp, int32_t d_hidden, int32_t n_layers,
+                      float beta, const float* g_sdf, float* g_enc, float* g_x, float* g_mlp,
+                      int32_t accumulate, void* workspace, size_t workspace_bytes, void* stream);
+int sn_mlp16_fwd_levels(const float* x, const float* enc, int32_t enc_dims, int64_t n_cap,
+                        const int32_t* n_dev, const float* mlp, int32_t d_hidden, int32_t n_layers,
+                        float beta, float* sdf, void* stream);
+int sn_mlp16_bwd_levels(const float* x, const float* enc, int32_t enc_dims, int64_t n_cap,
+                        const int32_t* n_dev, const float* mlp, int32_t d_hidden, int32_t n_layers,
+                        float beta, const float* g_sdf, float* g_enc, float* g_x, float* g_mlp,
+                        int32_t accumulate, void* ws, size_t ws_bytes, void* stream);
+
 /* ------------------------------------------------------------------------ */
 /* Fused patch rendering + losses, forward and backward: replaces the torch  */
 /* graph of models/renderer.py:142-276 (NeuS alpha, patch weights, 'dfd' or  */

@@ -55,8 +55,11 @@ SIGNATURES = {
     "sn_mlp_n_params": (C.c_int, [_i32, _i32, _i32]),
     "sn_mlp_bwd_workspace_bytes": (_sz, [_i64, _i32, _i32, _i32, _i32]),
     "sn_mlp_fwd": (C.c_int, [_p, _p, _i32, _i64, _p, _p, _i32, _i32, _f32, _p, _p, _p]),
+    "sn_mlp_fwd_levels": (C.c_int, [_p, _p, _i32, _i64, _p, _p, _i32, _i32, _f32, _p, _p, _p]),
     "sn_mlp_bwd": (C.c_int, [_p, _p, _i32, _i64, _p, _p, _i32, _i32, _f32, _p, _p, _p, _p,
                              _i32, _p, _sz, _p]),
+    "sn_mlp_bwd_levels": (C.c_int, [_p, _p, _i32, _i64, _p, _p, _i32, _i32, _f32, _p, _p, _p, _p,
+                                    _i32, _p, _sz, _p]),
     "sn_mlp_bwd_ad": (C.c_int, [_p, _p, _p, _p, _i32, _i64, _p, _p, _i32, _i32, _f32, _p, _p,
                                 _p, _p, _i32, _p, _sz, _p]),
     "sn_mlp_bwd_ad_enc": (C.c_int, [_p, _p, _p, _p, _i32, _i64, _p, _p, _i32, _i32, _f32, _p,
@@ -71,10 +74,13 @@ SIGNATURES = {
     "sn_adam_step": (C.c_int, [_p, _p, _p, _p, _i64, _f32, _p, C.c_double, C.c_double,
                                C.c_double, _i32, _p, _p]),
     "sn_mlp16_fwd": (C.c_int, [_p, _p, _i32, _i64, _p, _p, _i32, _i32, _f32, _p, _p]),
+    "sn_mlp16_fwd_levels": (C.c_int, [_p, _p, _i32, _i64, _p, _p, _i32, _i32, _f32, _p, _p]),
     "sn_mlp16_fwd_grad": (C.c_int, [_p, _p, _i32, _i64, _p, _p, _i32, _i32, _f32, _p, _p, _p]),
     "sn_mlp16_bwd_workspace_bytes": (_sz, [_i64, _i32, _i32, _i32]),
     "sn_mlp16_bwd": (C.c_int, [_p, _p, _i32, _i64, _p, _p, _i32, _i32, _f32, _p, _p, _p, _p,
                                _i32, _p, _sz, _p]),
+    "sn_mlp16_bwd_levels": (C.c_int, [_p, _p, _i32, _i64, _p, _p, _i32, _i32, _f32, _p, _p, _p, _p,
+                                      _i32, _p, _sz, _p]),
     "sn_render_step_set_impl": (None, [_i32]),
     "sn_ray_march_padded": (C.c_int, [_p, _p, _p, _p, _i32, _p, _p, _i32, _i32, _i32, _f32,
                                       _p, _f32, _i32, _p, _p, _p, _p]),
@@ -119,6 +125,8 @@ SIGNATURES = {
     "sn_hashgrid_bwd_bwd_dev": (C.c_int, [_p, _i64, _p, _p, _i32, _i32, _i32, _i32, _f32, _i32, _p, _p, _p, _p, _p, _p, _p]),
     "sn_hashgrid_tangent_dev": (C.c_int, [_p, _i64, _p, _p, _p, _i32, _i32, _i32, _i32, _f32, _i32, _p, _p, _p, _p]),
     "sn_hashgrid_bwd_ad_ws_dev": (C.c_int, [_p, _i64, _p, _p, _i32, _i32, _i32, _i32, _f32, _i32, _p, _p, _p, _p, _p, _p, _sz, _p]),
+    "sn_hashgrid_fwd_levels_dev": (C.c_int, [_p, _i64, _p, _p, _p, _i32, _i32, _i32, _f32, _i32,
+                                             _p, _p, _p]),
     "sn_occ_sample_workspace_bytes": (_sz, [_i32]),
     "sn_occ_sample_cells": (C.c_int, [_p, _i32, _p, _p, _p, _p, _p, _sz, _p]),
 }

@@ -291,6 +291,84 @@ hash_fwd_kernel(const float* __restrict__ x, int64_t n_cap, const int32_t* __res
     hash_fwd_point<F, TP, kPair>(i, x, params, d, na, enc);
 }
 
+// The encoding by levels, enc[l][i][2] (planes of n_cap points), F = 2: one
+// level per grid row, so that the chip works through one level's table at a
+// time -- 4 MB in fp32 at T = 2^19, an XCD's L2 -- where the row form above has
+// every level's in use at once (49 MB) and fetches a line per corner; and the
+// planes are written, and read by the MLP kernels, in whole lines.  The same
+// sums in the same order: the same bits as the rows.
+// kPts points per thread in flight.  kSplit: two neighbouring lanes per point,
+// one per x side of the cell, exchange the halves of their corners by DPP: the
+// x neighbours of the dense levels and every other one of the hashed levels
+// share a line, which one load instruction then fetches once.
+// us, rows -> levels: fp32 table, 2 M grid cells 1350 -> 570 (650 unsplit), 1.2 M
+// training points 204 -> 149 (163), 300 k 59 -> 43 (47), 30 k 18 -> 6.7 (8.1);
+// fp16 table (half the lines: the split's second lane costs more than it saves),
+// training points 1.2 M 164 -> 132 (145 split), 4 M at T = 2^21 670 -> 513 (557).
+template <typename TP, int kPts, bool kSplit>
+__global__ void __launch_bounds__(256)
+hash_fwd_levels_kernel(const float* __restrict__ x, int64_t n_cap,
+                       const int32_t* __restrict__ n_dev, const TP* __restrict__ params,
+                       HashGridDesc d, float* __restrict__ enc) {
+  typedef TP pair_t __attribute__((ext_vector_type(2)));
+  constexpr int kStep = kSplit ? 128 : 256, kCorners = kSplit ? 4 : 8;
+  const int64_t n = dev_count(n_cap, n_dev);
+  const int l = blockIdx.y;
+  const bool active = l < active_levels(d);
+  const pair_t* tab = reinterpret_cast<const pair_t*>(params + (int64_t)d.offset[l] * 2);
+  float* out = enc + (int64_t)l * n_cap * 2;
+  const int side = threadIdx.x & 1;  // kSplit: x side, and the feature summed
+  const int t = kSplit ? threadIdx.x >> 1 : threadIdx.x;
+  // (uniform bounds: the lanes of a pair stay together)
+  for (int64_t b = blockIdx.x * (int64_t)(kStep * kPts); b < n;
+       b += (int64_t)gridDim.x * kStep * kPts) {
+    float w[kPts][8];
+    pair_t v[kPts][kCorners];
+    if (active) {
+#pragma unroll
+      for (int u = 0; u < kPts; ++u) {
+        const int64_t i = min(b + u * kStep + t, n - 1);
+        const float p[3] = {x[3 * i], x[3 * i + 1], x[3 * i + 2]};
+        uint32_t idx[8];
+        float fr[3];
+        hg_level(p, d, l, idx, w[u], fr);
+#pragma unroll
+        for (int c = 0; c < kCorners; ++c)
+          v[u][c] = tab[kSplit ? (side ? idx[2 * c + 1] : idx[2 * c]) : idx[c]];
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < kPts; ++u) {
+      const int64_t i = b + u * kStep + t;
+      if constexpr (kSplit) {
+        float s = 0.f;
+        if (active) {
+#pragma unroll
+          for (int c = 0; c < 4; ++c) {
+            const float a0 = (float)v[u][c].x, a1 = (float)v[u][c].y;
+            const float mine = side ? a1 : a0, send = side ? a0 : a1;
+            const float got = __int_as_float(__builtin_amdgcn_update_dpp(
+                0, __float_as_int(send), 0xB1, 0xf, 0xf, true));  // quad_perm [1,0,3,2]
+            s += w[u][2 * c] * (side ? got : mine);
+            s += w[u][2 * c + 1] * (side ? mine : got);
+          }
+        }
+        if (i < n) out[2 * i + side] = s;
+      } else {
+        float s0 = 0.f, s1 = 0.f;
+        if (active) {
+#pragma unroll
+          for (int c = 0; c < 8; ++c) {
+            s0 += w[u][c] * (float)v[u][c].x;
+            s1 += w[u][c] * (float)v[u][c].y;
+          }
+        }
+        if (i < n) reinterpret_cast<float2*>(out)[i] = make_float2(s0, s1);
+      }
+    }
+  }
+}
+
 // The encoding's directional derivative along v (the tangent the double
 // backward of the analytic gradient needs, hash_bwd_bwd_kernel's grad_grad_enc):
 // out[l, f] = sum_c scale_l (v . d w_c / d frac) table_l[idx_c, f], from the
@@ -1461,6 +1539,35 @@ int sn_hashgrid_fwd16_dev(const float* x, int64_t n_cap, const int32_t* n_dev,
                                                               0, as_stream(stream)>>>(
                                 x, n_cap, n_dev, p16, d, enc)));
   return check_launch("sn_hashgrid_fwd16");
+}
+
+int sn_hashgrid_fwd_levels_dev(const float* x, int64_t n_cap, const int32_t* n_dev,
+                               const float* params, const void* params16, int32_t n_levels,
+                               int32_t log2_hashmap_size, int32_t base_resolution,
+                               float per_level_scale, int32_t n_active_levels,
+                               const int32_t* n_active_dev, float* enc, void* stream) {
+  clear_error();
+  HashGridDesc d;
+  int rc = hg_setup("sn_hashgrid_fwd_levels", n_levels, 2, log2_hashmap_size, base_resolution,
+                    per_level_scale, n_active_levels, &d);
+  if (rc) return rc;
+  d.n_active_dev = n_active_dev;
+  SN_REQUIRE(n_cap >= 0, "sn_hashgrid_fwd_levels: n < 0");
+  if (n_cap == 0) return SN_OK;
+  SN_REQUIRE(x && (params || params16) && enc, "sn_hashgrid_fwd_levels: null pointer");
+  SN_REQUIRE(reinterpret_cast<uintptr_t>(enc) % 8 == 0 &&
+                 reinterpret_cast<uintptr_t>(params) % 8 == 0 &&
+                 reinterpret_cast<uintptr_t>(params16) % 4 == 0,
+             "sn_hashgrid_fwd_levels: the table and enc hold aligned pairs");
+  // 16384 blocks of each level reach every point of 2^22; more are strided
+  const auto grid = [&](int per) { return dim3(grid_for(n_cap, per, 16384), n_levels); };
+  if (params16)
+    hash_fwd_levels_kernel<_Float16, 4, false><<<grid(1024), 256, 0, as_stream(stream)>>>(
+        x, n_cap, n_dev, reinterpret_cast<const _Float16*>(params16), d, enc);
+  else
+    hash_fwd_levels_kernel<float, 2, true><<<grid(256), 256, 0, as_stream(stream)>>>(
+        x, n_cap, n_dev, params, d, enc);
+  return check_launch("sn_hashgrid_fwd_levels");
 }
 
 int sn_hashgrid_dx_dev(const float* x, int64_t n_cap, const int32_t* n_dev, const float* params,

@@ -152,14 +152,22 @@ __device__ void load_weights(float* sw, const float* __restrict__ mlp, int E) {
 
 // The 4 input dims 16 kb + 4q .. +3 of point p, zero past n and past E + 3.
 // With vec4 (E % 4 == 0, 16-byte rows) they are encoding dims (one load), the
-// position, or padding; otherwise one guarded load per dim.
+// position, or padding; otherwise one guarded load per dim.  vec4 = 2: the
+// encoding by levels ([E / 2][n_cap][2], see hash_fwd_levels_kernel).
 __device__ __forceinline__ void load_in(const float* __restrict__ x, const float* __restrict__ enc,
-                                        int E, int vec4, int64_t p, bool ok, int c4,
+                                        int E, int vec4, int64_t n_cap, int64_t p, bool ok, int c4,
                                         float (&v)[4]) {
   if (vec4) {
     float4 a = {0.f, 0.f, 0.f, 0.f};
-    if (ok && c4 < E) a = *reinterpret_cast<const float4*>(enc + p * E + c4);
-    else if (ok && c4 == E) a = float4{x[p * 3], x[p * 3 + 1], x[p * 3 + 2], 0.f};
+    if (ok && c4 < E) {
+      if (vec4 == 2) {
+        const float2* e2 = reinterpret_cast<const float2*>(enc) + (int64_t)(c4 >> 1) * n_cap + p;
+        const float2 lo = e2[0], hi = e2[n_cap];
+        a = float4{lo.x, lo.y, hi.x, hi.y};
+      } else {
+        a = *reinterpret_cast<const float4*>(enc + p * E + c4);
+      }
+    } else if (ok && c4 == E) a = float4{x[p * 3], x[p * 3 + 1], x[p * 3 + 2], 0.f};
     v[0] = a.x;
     v[1] = a.y;
     v[2] = a.z;
@@ -273,7 +281,7 @@ mlp_fwd_kernel(const float* __restrict__ x, const float* __restrict__ enc, int E
     asm volatile("" : "+v"(qs), "+s"(Es), "+s"(v4s));
     float h0[KB][4];
 #pragma unroll
-    for (int kb = 0; kb < KB; ++kb) load_in(x, enc, Es, v4s, p, ok, 16 * kb + 4 * qs, h0[kb]);
+    for (int kb = 0; kb < KB; ++kb) load_in(x, enc, Es, v4s, n_cap, p, ok, 16 * kb + 4 * qs, h0[kb]);
     floatx4 z[MB];
     init_bias<MB>(vec, z);
     gemm<MB, KB>(smem, M::LD0, h0, z);
@@ -491,7 +499,7 @@ mlp_bwd_kernel(const float* __restrict__ x, const float* __restrict__ enc, int E
     asm volatile("" : "+v"(qs), "+s"(Es), "+s"(v4s));
     float h0[KB][4];
 #pragma unroll
-    for (int kb = 0; kb < KB; ++kb) load_in(x, enc, Es, v4s, p, ok, 16 * kb + 4 * qs, h0[kb]);
+    for (int kb = 0; kb < KB; ++kb) load_in(x, enc, Es, v4s, n_cap, p, ok, 16 * kb + 4 * qs, h0[kb]);
     const float gs = ok ? g_sdf[p] : 0.f;
     if (q == 0) dbo += gs;
     floatx4 z[MB];
@@ -612,11 +620,11 @@ mlp_bwd_ad_kernel(const float* __restrict__ x, const float* __restrict__ enc,
     {
       float h0[KB][4];
 #pragma unroll
-      for (int kb = 0; kb < KB; ++kb) load_in(x, enc, Es, v4s, p, ok, 16 * kb + 4 * qs, h0[kb]);
+      for (int kb = 0; kb < KB; ++kb) load_in(x, enc, Es, v4s, n_cap, p, ok, 16 * kb + 4 * qs, h0[kb]);
       init_bias<MB>(vec, z);
       gemm<MB, KB>(smem, M::LD0, h0, z);
 #pragma unroll
-      for (int kb = 0; kb < KB; ++kb) load_in(v, encd, Es, v4s, p, ok, 16 * kb + 4 * qs, h0[kb]);
+      for (int kb = 0; kb < KB; ++kb) load_in(v, encd, Es, v4s, n_cap, p, ok, 16 * kb + 4 * qs, h0[kb]);
       init_zero<MB>(zd);
       gemm<MB, KB>(smem, M::LD0, h0, zd);
     }
@@ -690,7 +698,7 @@ mlp_bwd_ad_kernel(const float* __restrict__ x, const float* __restrict__ enc,
       float h0[KB][4];
 #pragma unroll
       for (int kb = 0; kb < KB; ++kb)
-        load_in(pass ? v : x, pass ? encd : enc, Es, v4s, p, ok, 16 * kb + 4 * qs, h0[kb]);
+        load_in(pass ? v : x, pass ? encd : enc, Es, v4s, n_cap, p, ok, 16 * kb + 4 * qs, h0[kb]);
       tile_store<TP, MB>(tA, pass ? gt : gb);
       tile_store<TP, KB>(tB, h0);
       __syncthreads();
@@ -840,9 +848,12 @@ size_t sn_mlp_bwd_workspace_bytes(int64_t n_cap, int32_t enc_dims, int32_t d_hid
   return (size_t)grid_blocks(n_cap, kBwdBlocksMax) * np * sizeof(float);
 }
 
-int sn_mlp_fwd(const float* x, const float* enc, int32_t enc_dims, int64_t n_cap,
-               const int32_t* n_dev, const float* mlp, int32_t d_hidden, int32_t n_layers,
-               float beta, float* sdf, float* dsdf_dh0, void* stream) {
+}  // extern "C"
+
+template <bool kLevels>
+static int mlp_fwd_impl(const float* x, const float* enc, int32_t enc_dims, int64_t n_cap,
+                        const int32_t* n_dev, const float* mlp, int32_t d_hidden, int32_t n_layers,
+                        float beta, float* sdf, float* dsdf_dh0, void* stream) {
   clear_error();
   MlpCfg c;
   int rc = mlp_cfg("sn_mlp_fwd", enc_dims, d_hidden, n_layers, &c);
@@ -852,7 +863,11 @@ int sn_mlp_fwd(const float* x, const float* enc, int32_t enc_dims, int64_t n_cap
   SN_REQUIRE(x && mlp && sdf && (enc || enc_dims == 0), "sn_mlp_fwd: null pointer");
   hipStream_t s = as_stream(stream);
   const unsigned grid = grid_blocks(n_cap, kFwdBlocksMax);
-  const int v4 = vec4_ok(enc, enc_dims);
+  int v4 = vec4_ok(enc, enc_dims);
+  if (kLevels) {
+    SN_REQUIRE(v4, "sn_mlp_fwd: a levels encoding has E % 4 == 0 and is 16-byte aligned");
+    v4 = 2;
+  }
   SN_MLP_DISPATCH(c, {
     constexpr size_t sm = sizeof(float) * Mlp<kH, kNH, kKB>::kFwd;
     if (dsdf_dh0)
@@ -865,10 +880,29 @@ int sn_mlp_fwd(const float* x, const float* enc, int32_t enc_dims, int64_t n_cap
   return check_launch("sn_mlp_fwd");
 }
 
-int sn_mlp_bwd(const float* x, const float* enc, int32_t enc_dims, int64_t n_cap,
+extern "C" {
+
+int sn_mlp_fwd(const float* x, const float* enc, int32_t enc_dims, int64_t n_cap,
                const int32_t* n_dev, const float* mlp, int32_t d_hidden, int32_t n_layers,
-               float beta, const float* g_sdf, float* g_enc, float* g_x, float* g_mlp,
-               int32_t accumulate, void* workspace, size_t workspace_bytes, void* stream) {
+               float beta, float* sdf, float* dsdf_dh0, void* stream) {
+  return mlp_fwd_impl<false>(
+      x, enc, enc_dims, n_cap, n_dev, mlp, d_hidden, n_layers, beta, sdf, dsdf_dh0, stream);
+}
+
+int sn_mlp_fwd_levels(const float* x, const float* enc, int32_t enc_dims, int64_t n_cap,
+                      const int32_t* n_dev, const float* mlp, int32_t d_hidden, int32_t n_layers,
+                      float beta, float* sdf, float* dsdf_dh0, void* stream) {
+  return mlp_fwd_impl<true>(
+      x, enc, enc_dims, n_cap, n_dev, mlp, d_hidden, n_layers, beta, sdf, dsdf_dh0, stream);
+}
+
+}  // extern "C"
+
+template <bool kLevels>
+static int mlp_bwd_impl(const float* x, const float* enc, int32_t enc_dims, int64_t n_cap,
+                        const int32_t* n_dev, const float* mlp, int32_t d_hidden, int32_t n_layers,
+                        float beta, const float* g_sdf, float* g_enc, float* g_x, float* g_mlp,
+                        int32_t accumulate, void* workspace, size_t workspace_bytes, void* stream) {
   clear_error();
   MlpCfg c;
   int rc = mlp_cfg("sn_mlp_bwd", enc_dims, d_hidden, n_layers, &c);
@@ -884,7 +918,11 @@ int sn_mlp_bwd(const float* x, const float* enc, int32_t enc_dims, int64_t n_cap
   const int np = sn_mlp_n_params(c.d, d_hidden, n_layers);
   const unsigned grid = grid_blocks(n_cap, kBwdBlocksMax);
   float* part = reinterpret_cast<float*>(workspace);
-  const int v4 = vec4_ok(enc, enc_dims) && vec4_ok(g_enc, enc_dims);
+  int v4 = vec4_ok(enc, enc_dims) && vec4_ok(g_enc, enc_dims);
+  if (kLevels) {
+    SN_REQUIRE(v4, "sn_mlp_bwd: a levels encoding has E % 4 == 0 and is 16-byte aligned");
+    v4 = 2;
+  }
   SN_MLP_DISPATCH(c, {
     constexpr size_t sm = sizeof(float) * Mlp<kH, kNH, kKB>::kBwd;
     allow_smem(mlp_bwd_kernel<kH, kNH, kKB>, sm);
@@ -893,6 +931,26 @@ int sn_mlp_bwd(const float* x, const float* enc, int32_t enc_dims, int64_t n_cap
   });
   if ((rc = mlp_reduce_rows(part, (int64_t)grid, np, g_mlp, accumulate, s))) return rc;
   return check_launch("sn_mlp_bwd");
+}
+
+extern "C" {
+
+int sn_mlp_bwd(const float* x, const float* enc, int32_t enc_dims, int64_t n_cap,
+               const int32_t* n_dev, const float* mlp, int32_t d_hidden, int32_t n_layers,
+               float beta, const float* g_sdf, float* g_enc, float* g_x, float* g_mlp,
+               int32_t accumulate, void* workspace, size_t workspace_bytes, void* stream) {
+  return mlp_bwd_impl<false>(
+      x, enc, enc_dims, n_cap, n_dev, mlp, d_hidden, n_layers, beta, g_sdf, g_enc, g_x, g_mlp,
+      accumulate, workspace, workspace_bytes, stream);
+}
+
+int sn_mlp_bwd_levels(const float* x, const float* enc, int32_t enc_dims, int64_t n_cap,
+                      const int32_t* n_dev, const float* mlp, int32_t d_hidden, int32_t n_layers,
+                      float beta, const float* g_sdf, float* g_enc, float* g_x, float* g_mlp,
+                      int32_t accumulate, void* workspace, size_t workspace_bytes, void* stream) {
+  return mlp_bwd_impl<true>(
+      x, enc, enc_dims, n_cap, n_dev, mlp, d_hidden, n_layers, beta, g_sdf, g_enc, g_x, g_mlp,
+      accumulate, workspace, workspace_bytes, stream);
 }
 
 static int mlp_bwd_ad(const float* x, const float* enc, const float* v, const float* enc_dot,

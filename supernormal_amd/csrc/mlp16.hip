@@ -183,8 +183,8 @@ __device__ void build_frags(char* smem, const float* __restrict__ mlp, int E) {
 // them, or padding; otherwise one guarded load per slot.
 // `one` is the value of the constant slot: 1 for h0, 0 for a tangent of h0.
 __device__ __forceinline__ void load_h0(const float* __restrict__ x, const float* __restrict__ enc,
-                                        int E, bool vec4, int64_t p, bool ok, int kb, int q,
-                                        float (&v)[8], float one = 1.f) {
+                                        int E, int vec4, int64_t n_cap, int64_t p, bool ok, int kb,
+                                        int q, float (&v)[8], float one = 1.f) {
   const int c0 = 32 * kb + 8 * q;
   if (vec4) {
 #pragma unroll
@@ -192,7 +192,13 @@ __device__ __forceinline__ void load_h0(const float* __restrict__ x, const float
       const int c4 = c0 + 4 * h;
       float4 a = {0.f, 0.f, 0.f, 0.f};
       if (ok && c4 < E) {
-        a = *reinterpret_cast<const float4*>(enc + p * E + c4);
+        if (vec4 == 2) {  // by levels: [E / 2][n_cap][2] (hash_fwd_levels_kernel)
+          const float2* e2 = reinterpret_cast<const float2*>(enc) + (int64_t)(c4 >> 1) * n_cap + p;
+          const float2 lo = e2[0], hi = e2[n_cap];
+          a = float4{lo.x, lo.y, hi.x, hi.y};
+        } else {
+          a = *reinterpret_cast<const float4*>(enc + p * E + c4);
+        }
       } else if (ok && c4 == E) {
         a = float4{x[p * 3], x[p * 3 + 1], x[p * 3 + 2], one};
       }
@@ -354,9 +360,11 @@ mlp16_fwd_kernel(const float* __restrict__ x, const float* __restrict__ enc, int
     asm volatile("" ::: "memory");
     const int64_t p = g * 16 + r;
     const bool ok = p < n;
+    int qs = q, Es = E, v4s = vec4;  // opaque: see mlp16_bwd_kernel
+    asm volatile("" : "+v"(qs), "+s"(Es), "+s"(v4s));
     float h0[KB0][8];
 #pragma unroll
-    for (int kb = 0; kb < KB0; ++kb) load_h0(x, enc, E, vec4, p, ok, kb, q, h0[kb]);
+    for (int kb = 0; kb < KB0; ++kb) load_h0(x, enc, Es, v4s, n_cap, p, ok, kb, qs, h0[kb]);
     Fwd<H, NH, KB0> F;
     float s = 0.f;
     forward_group<H, NH, KB0, false, true>(
@@ -407,7 +415,7 @@ mlp16_fwd_grad_kernel(const float* __restrict__ x, const float* __restrict__ enc
     asm volatile("" : "+v"(qs), "+s"(Es), "+s"(v4s));
     float h0[KB0][8];
 #pragma unroll
-    for (int kb = 0; kb < KB0; ++kb) load_h0(x, enc, Es, v4s, p, ok, kb, qs, h0[kb]);
+    for (int kb = 0; kb < KB0; ++kb) load_h0(x, enc, Es, v4s, n_cap, p, ok, kb, qs, h0[kb]);
     Fwd<H, NH, KB0> F;
     float s = 0.f, gz[MB][4];
     forward_group<H, NH, KB0, true, true>(
@@ -623,7 +631,7 @@ mlp16_bwd_kernel(const float* __restrict__ x, const float* __restrict__ enc, int
     asm volatile("" : "+v"(qs), "+s"(Es), "+s"(v4s));
     float h0[KB0][8];
 #pragma unroll
-    for (int kb = 0; kb < KB0; ++kb) load_h0(x, enc, Es, v4s, p, ok, kb, qs, h0[kb]);
+    for (int kb = 0; kb < KB0; ++kb) load_h0(x, enc, Es, v4s, n_cap, p, ok, kb, qs, h0[kb]);
     const float gs = ok ? g_sdf[p] : 0.f;
     Fwd<H, NH, KB0> F;
     if (q == 0) dbo += gs;
@@ -790,8 +798,8 @@ mlp16_bwd_ad_kernel(const float* __restrict__ x, const float* __restrict__ enc,
       float h0[KB0][8], hd0[KB0][8];
 #pragma unroll
       for (int kb = 0; kb < KB0; ++kb) {
-        load_h0(x, enc, Es, v4s, p, ok, kb, qs, h0[kb]);
-        load_h0(v, encd, Es, v4s, p, ok, kb, qs, hd0[kb], 0.f);
+        load_h0(x, enc, Es, v4s, n_cap, p, ok, kb, qs, h0[kb]);
+        load_h0(v, encd, Es, v4s, n_cap, p, ok, kb, qs, hd0[kb], 0.f);
       }
 #pragma unroll
       for (int kb = 0; kb < KB0; ++kb)
@@ -913,8 +921,8 @@ mlp16_bwd_ad_kernel(const float* __restrict__ x, const float* __restrict__ enc,
       float h0[KB0][8], hd0[KB0][8];
 #pragma unroll
       for (int kb = 0; kb < KB0; ++kb) {
-        load_h0(x, enc, Es, v4s, p, ok, kb, qs, h0[kb]);
-        load_h0(v, encd, Es, v4s, p, ok, kb, qs, hd0[kb], 0.f);
+        load_h0(x, enc, Es, v4s, n_cap, p, ok, kb, qs, h0[kb]);
+        load_h0(v, encd, Es, v4s, n_cap, p, ok, kb, qs, hd0[kb], 0.f);
       }
 #pragma unroll
       for (int kb = 0; kb < KB0; ++kb)
@@ -1027,9 +1035,12 @@ using namespace sn::m16;
 
 extern "C" {
 
-int sn_mlp16_fwd(const float* x, const float* enc, int32_t enc_dims, int64_t n_cap,
-                 const int32_t* n_dev, const float* mlp, int32_t d_hidden, int32_t n_layers,
-                 float beta, float* sdf, void* stream) {
+}  // extern "C"
+
+template <bool kLevels>
+static int mlp16_fwd_impl(const float* x, const float* enc, int32_t enc_dims, int64_t n_cap,
+                          const int32_t* n_dev, const float* mlp, int32_t d_hidden, int32_t n_layers,
+                          float beta, float* sdf, void* stream) {
   clear_error();
   int kb0 = 0;
   int rc = check_cfg("sn_mlp16_fwd", enc_dims, d_hidden, n_layers, &kb0);
@@ -1037,15 +1048,36 @@ int sn_mlp16_fwd(const float* x, const float* enc, int32_t enc_dims, int64_t n_c
   SN_REQUIRE(n_cap >= 0 && beta > 0.f, "sn_mlp16_fwd: bad n / beta");
   if (n_cap == 0) return SN_OK;
   SN_REQUIRE(x && mlp && sdf && (enc || enc_dims == 0), "sn_mlp16_fwd: null pointer");
+  int v4 = vec4_ok(enc, enc_dims);
+  if (kLevels) {
+    SN_REQUIRE(v4, "sn_mlp16_fwd: a levels encoding has E % 4 == 0 and is 16-byte aligned");
+    v4 = 2;
+  }
   const unsigned grid = blocks_for(n_cap, kFwdBlocksMax);
   hipStream_t s = as_stream(stream);
   SN_MLP16_DISPATCH(d_hidden, n_layers, kb0, {
     constexpr size_t lds = Cfg<kH, kNH, kKB>::fwd_lds;
     allow_lds(mlp16_fwd_kernel<kH, kNH, kKB>, lds);
     mlp16_fwd_kernel<kH, kNH, kKB><<<grid, 64 * kWaves, lds, s>>>(
-        x, enc, enc_dims, vec4_ok(enc, enc_dims), n_cap, n_dev, mlp, beta, sdf);
+        x, enc, enc_dims, v4, n_cap, n_dev, mlp, beta, sdf);
   });
   return check_launch("sn_mlp16_fwd");
+}
+
+extern "C" {
+
+int sn_mlp16_fwd(const float* x, const float* enc, int32_t enc_dims, int64_t n_cap,
+                 const int32_t* n_dev, const float* mlp, int32_t d_hidden, int32_t n_layers,
+                 float beta, float* sdf, void* stream) {
+  return mlp16_fwd_impl<false>(
+      x, enc, enc_dims, n_cap, n_dev, mlp, d_hidden, n_layers, beta, sdf, stream);
+}
+
+int sn_mlp16_fwd_levels(const float* x, const float* enc, int32_t enc_dims, int64_t n_cap,
+                        const int32_t* n_dev, const float* mlp, int32_t d_hidden, int32_t n_layers,
+                        float beta, float* sdf, void* stream) {
+  return mlp16_fwd_impl<true>(
+      x, enc, enc_dims, n_cap, n_dev, mlp, d_hidden, n_layers, beta, sdf, stream);
 }
 
 int sn_mlp16_fwd_grad(const float* x, const float* enc, int32_t enc_dims, int64_t n_cap,
@@ -1076,10 +1108,13 @@ size_t sn_mlp16_bwd_workspace_bytes(int64_t n_cap, int32_t enc_dims, int32_t d_h
   return (size_t)blocks_for(n_cap, kBwdBlocksMax) * np * sizeof(float);
 }
 
-int sn_mlp16_bwd(const float* x, const float* enc, int32_t enc_dims, int64_t n_cap,
-                 const int32_t* n_dev, const float* mlp, int32_t d_hidden, int32_t n_layers,
-                 float beta, const float* g_sdf, float* g_enc, float* g_x, float* g_mlp,
-                 int32_t accumulate, void* ws, size_t ws_bytes, void* stream) {
+}  // extern "C"
+
+template <bool kLevels>
+static int mlp16_bwd_impl(const float* x, const float* enc, int32_t enc_dims, int64_t n_cap,
+                          const int32_t* n_dev, const float* mlp, int32_t d_hidden, int32_t n_layers,
+                          float beta, const float* g_sdf, float* g_enc, float* g_x, float* g_mlp,
+                          int32_t accumulate, void* ws, size_t ws_bytes, void* stream) {
   clear_error();
   int kb0 = 0;
   int rc = check_cfg("sn_mlp16_bwd", enc_dims, d_hidden, n_layers, &kb0);
@@ -1098,17 +1133,41 @@ int sn_mlp16_bwd(const float* x, const float* enc, int32_t enc_dims, int64_t n_c
     set_error("sn_mlp16_bwd: workspace %zu < %zu bytes", ws_bytes, need);
     return SN_ESPACE;
   }
+  int v4 = vec4_ok(enc, enc_dims) && vec4_ok(g_enc, enc_dims);
+  if (kLevels) {
+    SN_REQUIRE(v4, "sn_mlp16_bwd: a levels encoding has E % 4 == 0 and is 16-byte aligned");
+    v4 = 2;
+  }
   const unsigned grid = blocks_for(n_cap, kBwdBlocksMax);
   float* part = reinterpret_cast<float*>(ws);
   SN_MLP16_DISPATCH(d_hidden, n_layers, kb0, {
     constexpr size_t lds = Cfg<kH, kNH, kKB>::bwd_lds;
     allow_lds(mlp16_bwd_kernel<kH, kNH, kKB>, lds);
     mlp16_bwd_kernel<kH, kNH, kKB><<<grid, 64 * kWaves, lds, s>>>(
-        x, enc, enc_dims, vec4_ok(enc, enc_dims) && vec4_ok(g_enc, enc_dims), n_cap, n_dev, mlp,
-        beta, g_sdf, g_enc, g_x, part);
+        x, enc, enc_dims, v4, n_cap, n_dev, mlp, beta, g_sdf, g_enc, g_x, part);
   });
   if ((rc = check_launch("sn_mlp16_bwd"))) return rc;
   return mlp_reduce_rows(part, (int64_t)grid, np, g_mlp, accumulate, s);
+}
+
+extern "C" {
+
+int sn_mlp16_bwd(const float* x, const float* enc, int32_t enc_dims, int64_t n_cap,
+                 const int32_t* n_dev, const float* mlp, int32_t d_hidden, int32_t n_layers,
+                 float beta, const float* g_sdf, float* g_enc, float* g_x, float* g_mlp,
+                 int32_t accumulate, void* ws, size_t ws_bytes, void* stream) {
+  return mlp16_bwd_impl<false>(
+      x, enc, enc_dims, n_cap, n_dev, mlp, d_hidden, n_layers, beta, g_sdf, g_enc, g_x, g_mlp,
+      accumulate, ws, ws_bytes, stream);
+}
+
+int sn_mlp16_bwd_levels(const float* x, const float* enc, int32_t enc_dims, int64_t n_cap,
+                        const int32_t* n_dev, const float* mlp, int32_t d_hidden, int32_t n_layers,
+                        float beta, const float* g_sdf, float* g_enc, float* g_x, float* g_mlp,
+                        int32_t accumulate, void* ws, size_t ws_bytes, void* stream) {
+  return mlp16_bwd_impl<true>(
+      x, enc, enc_dims, n_cap, n_dev, mlp, d_hidden, n_layers, beta, g_sdf, g_enc, g_x, g_mlp,
+      accumulate, ws, ws_bytes, stream);
 }
 
 int sn_mlp16_bwd_ad_enc(const float* x, const float* enc, const float* v, const float* enc_dot,

@@ -36,6 +36,9 @@ class SDFConfig:
         self.n_layers = int(n_layers)
         self.beta = float(beta)
         self.E = grid["n_levels"] * grid["n_features"]
+        # the sdf's encoding by levels [L, N, 2] rather than by rows [N, E]
+        # (the analytic gradient's kernels take rows)
+        self.level_pairs = grid["n_features"] == 2 and self.E % 4 == 0
         # 'fp16': MLP on the fp16/bf16 matrix cores (sn_mlp16_*) for the sdf
         # value and its backward; the analytic gradient stays on fp32 kernels
         self.precision = precision
@@ -45,6 +48,9 @@ class SDFConfig:
 
     def ws(self, n_active, n, device):
         return self.workspace.get(self.hash_args(n_active), n, device)
+
+    def by_levels(self, params):
+        return self.level_pairs and params.data_ptr() % 8 == 0
 
     def hash_args(self, n_active):
         g = self.grid
@@ -57,7 +63,13 @@ def pack_mlp(layers):
     return torch.cat([t.reshape(-1) for W, b in layers for t in (W, b)])
 
 
-def _hash_fwd(cfg, x, params, n_active, n_dev=None):
+def _hash_fwd(cfg, x, params, n_active, by_levels=False):
+    if by_levels:
+        enc = torch.empty((cfg.E // 2, x.shape[0], 2), dtype=torch.float32, device=x.device)
+        L, _, *rest = cfg.hash_args(n_active)
+        call("sn_hashgrid_fwd_levels_dev", ptr(x), x.shape[0], None, ptr(params), None, L, *rest,
+             None, ptr(enc), stream_of(x.device))
+        return enc
     enc = torch.empty((x.shape[0], cfg.E), dtype=torch.float32, device=x.device)
     call("sn_hashgrid_fwd", ptr(x), x.shape[0], ptr(params), *cfg.hash_args(n_active), ptr(enc),
          stream_of(x.device))
@@ -66,13 +78,14 @@ def _hash_fwd(cfg, x, params, n_active, n_dev=None):
 
 def _mlp_fwd(cfg, x, enc, mlp, want_dh0):
     n = x.shape[0]
+    lv = "_levels" if enc.dim() == 3 else ""
     sdf = torch.empty(n, dtype=torch.float32, device=x.device)
     if cfg.precision == "fp16" and not want_dh0:
-        call("sn_mlp16_fwd", ptr(x), ptr(enc), cfg.E, n, None, ptr(mlp), cfg.d_hidden,
+        call("sn_mlp16_fwd" + lv, ptr(x), ptr(enc), cfg.E, n, None, ptr(mlp), cfg.d_hidden,
              cfg.n_layers, cfg.beta, ptr(sdf), stream_of(x.device))
         return sdf, None
     dh0 = torch.empty((n, 3 + cfg.E), dtype=torch.float32, device=x.device) if want_dh0 else None
-    call("sn_mlp_fwd", ptr(x), ptr(enc), cfg.E, n, None, ptr(mlp), cfg.d_hidden, cfg.n_layers,
+    call("sn_mlp_fwd" + lv, ptr(x), ptr(enc), cfg.E, n, None, ptr(mlp), cfg.d_hidden, cfg.n_layers,
          cfg.beta, ptr(sdf), ptr(dh0), stream_of(x.device))
     return sdf, dh0
 
@@ -81,7 +94,7 @@ class _SDFFn(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, params, mlp, cfg, n_active):
         x = x.contiguous()
-        enc = _hash_fwd(cfg, x, params, n_active)
+        enc = _hash_fwd(cfg, x, params, n_active, cfg.by_levels(params))
         sdf, _ = _mlp_fwd(cfg, x, enc, mlp, False)
         ctx.save_for_backward(x, enc, params, mlp)
         ctx.cfg, ctx.n_active = cfg, n_active
@@ -100,16 +113,17 @@ class _SDFFn(torch.autograd.Function):
         g_mlp = torch.empty_like(mlp)
         lib = _lib.lib()
         s = stream_of(dev)
+        lv = "_levels" if enc.dim() == 3 else ""
         if cfg.precision == "fp16":
             ws = workspace(lib.sn_mlp16_bwd_workspace_bytes(n, cfg.E, cfg.d_hidden,
                                                             cfg.n_layers), dev)
-            call("sn_mlp16_bwd", ptr(x), ptr(enc), cfg.E, n, None, ptr(mlp), cfg.d_hidden,
+            call("sn_mlp16_bwd" + lv, ptr(x), ptr(enc), cfg.E, n, None, ptr(mlp), cfg.d_hidden,
                  cfg.n_layers, cfg.beta, ptr(g_sdf), ptr(g_enc), None, ptr(g_mlp), 0, ptr(ws),
                  ws.numel(), s)
         else:
             ws = workspace(lib.sn_mlp_bwd_workspace_bytes(n, cfg.E, cfg.d_hidden, cfg.n_layers,
                                                           0), dev)
-            call("sn_mlp_bwd", ptr(x), ptr(enc), cfg.E, n, None, ptr(mlp), cfg.d_hidden,
+            call("sn_mlp_bwd" + lv, ptr(x), ptr(enc), cfg.E, n, None, ptr(mlp), cfg.d_hidden,
                  cfg.n_layers, cfg.beta, ptr(g_sdf), ptr(g_enc), None, ptr(g_mlp), 0, ptr(ws),
                  ws.numel(), s)
         g_params = torch.zeros_like(params)

@@ -339,7 +339,13 @@ class SyncFreeStep:
 
     def _sdf_fwd(self, pts, enc, sdf, cap, n_dev, mlp, s):
         cfg = self.cfg
-        if self.table16 is not None:
+        lv = "_levels" if cfg.by_levels(self.net.encoding.params) else ""
+        if lv:
+            L, _, *rest = self._hash_args()
+            call("sn_hashgrid_fwd_levels_dev", ptr(pts), cap, ptr(n_dev),
+                 ptr(self.net.encoding.params), ptr(self.table16), L, *rest,
+                 ptr(self.levels_dev), ptr(enc), s)
+        elif self.table16 is not None:
             call("sn_hashgrid_fwd16_dev", ptr(pts), cap, ptr(n_dev), ptr(self.table16),
                  *self._hash_args(), ptr(self.levels_dev), ptr(enc), s)
         else:
@@ -347,10 +353,10 @@ class SyncFreeStep:
                  ptr(self.net.encoding.params), *self._hash_args(), ptr(self.levels_dev),
                  ptr(enc), s)
         if self.precision == "fp16":
-            call("sn_mlp16_fwd", ptr(pts), ptr(enc), cfg.E, cap, ptr(n_dev), ptr(mlp),
+            call("sn_mlp16_fwd" + lv, ptr(pts), ptr(enc), cfg.E, cap, ptr(n_dev), ptr(mlp),
                  cfg.d_hidden, cfg.n_layers, cfg.beta, ptr(sdf), s)
         else:
-            call("sn_mlp_fwd", ptr(pts), ptr(enc), cfg.E, cap, ptr(n_dev), ptr(mlp),
+            call("sn_mlp_fwd" + lv, ptr(pts), ptr(enc), cfg.E, cap, ptr(n_dev), ptr(mlp),
                  cfg.d_hidden, cfg.n_layers, cfg.beta, ptr(sdf), None, s)
 
     def _iteration(self, inputs=None):
@@ -433,15 +439,16 @@ class SyncFreeStep:
              ptr(self.g_sdf), None, ptr(self.g_grad) if ad else None, ptr(self.losses),
              ptr(self.partials), None, None, s)
         # backward: the MLP here; the hash grid in its own part (_part_hash)
+        lv = "_levels" if cfg.by_levels(self.net.encoding.params) else ""
         if ad:
             self._ad_backward(c1, mlp_d, s)
         elif self.precision == "fp16":
-            call("sn_mlp16_bwd", ptr(self.pts), ptr(self.enc), cfg.E, c1, ptr(self.ne),
+            call("sn_mlp16_bwd" + lv, ptr(self.pts), ptr(self.enc), cfg.E, c1, ptr(self.ne),
                  ptr(mlp_d), cfg.d_hidden, cfg.n_layers, cfg.beta, ptr(self.g_sdf),
                  ptr(self.g_enc), None, ptr(self.g_mlp), 0, ptr(self.ws_mlp),
                  self.ws_mlp.numel(), s)
         else:
-            call("sn_mlp_bwd", ptr(self.pts), ptr(self.enc), cfg.E, c1, ptr(self.ne),
+            call("sn_mlp_bwd" + lv, ptr(self.pts), ptr(self.enc), cfg.E, c1, ptr(self.ne),
                  ptr(mlp_d), cfg.d_hidden, cfg.n_layers, cfg.beta, ptr(self.g_sdf),
                  ptr(self.g_enc), None, ptr(self.g_mlp), 0, ptr(self.ws_mlp),
                  self.ws_mlp.numel(), s)
