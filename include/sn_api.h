@@ -195,6 +195,12 @@ int sn_mlp_pack_fwd(const float* flat, int32_t n_layers, const int64_t* layers, 
 int sn_mlp_pack_bwd(const float* flat, int32_t n_layers, const int64_t* layers,
                     const float* g_packed, float* grad, const float* variance,
                     const float* g_inv_s, float* g_variance, void* stream);
+/* The same for parameters that are tensors of their own: `layers` holds the  */
+/* addresses of v, g (0: no weight norm) and b in place of the offsets, and  */
+/* the gradients are set (not added) in grad, [dv | dg | db] layer by layer. */
+int sn_mlp_pack_tensors_fwd(int32_t n_layers, const int64_t* layers, float* packed, void* stream);
+int sn_mlp_pack_tensors_bwd(int32_t n_layers, const int64_t* layers, const float* g_packed,
+                            float* grad, void* stream);
 /* As sn_ray_march_padded, reading occupancy from 4x4x4 brick masks (built  */
 /* by sn_occ_pack_bricks from `grid`; NULL: the byte grid): one 8-byte read */
 /* serves the 64 cells of a brick.  Same samples.  No counterpart in the    */

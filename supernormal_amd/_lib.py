@@ -127,6 +127,8 @@ SIGNATURES = {
     "sn_hashgrid_bwd_ad_ws_dev": (C.c_int, [_p, _i64, _p, _p, _i32, _i32, _i32, _i32, _f32, _i32, _p, _p, _p, _p, _p, _p, _sz, _p]),
     "sn_hashgrid_fwd_levels_dev": (C.c_int, [_p, _i64, _p, _p, _p, _i32, _i32, _i32, _f32, _i32,
                                              _p, _p, _p]),
+    "sn_mlp_pack_tensors_fwd": (C.c_int, [_i32, _p, _p, _p]),
+    "sn_mlp_pack_tensors_bwd": (C.c_int, [_i32, _p, _p, _p, _p]),
     "sn_occ_sample_workspace_bytes": (_sz, [_i32]),
     "sn_occ_sample_cells": (C.c_int, [_p, _i32, _p, _p, _p, _p, _p, _sz, _p]),
 }

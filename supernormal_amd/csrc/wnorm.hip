@@ -4,9 +4,10 @@
 // variance's inv_s = clip(exp(10 * variance), 1e-6, 1e6) (fields.py:133-139).
 //
 // Packed layout (as pack_mlp): per layer W [out, in] row-major, then b [out].
-// Parameters and their gradients live in one flat buffer each; a layer
+// Parameters and their gradients live in one flat buffer each, where a layer
 // names its tensors by offsets into them (v, g, b; g < 0: no weight norm,
-// W = v).  One wavefront per weight row: the row's squared norm is a
+// W = v) and gradients are added to, or the parameters are tensors of their
+// own and the gradients are set in one buffer, [dv | dg | db] per layer.  One wavefront per weight row: the row's squared norm is a
 // wavefront sum; the backward is
 //   dL/dg[r]  += sum_i dW[r,i] v[r,i] / n_r
 //   dL/dv[r,i] += (g[r] / n_r) * (dW[r,i] - v[r,i] * (sum_j dW[r,j] v[r,j]) / n_r^2)
@@ -19,7 +20,9 @@ constexpr int kMaxPackLayers = 8;
 
 struct PackLayers {
   int32_t n;
-  int64_t v[kMaxPackLayers], g[kMaxPackLayers], b[kMaxPackLayers], packed[kMaxPackLayers];
+  const float *v[kMaxPackLayers], *g[kMaxPackLayers], *b[kMaxPackLayers];
+  float *dv[kMaxPackLayers], *dg[kMaxPackLayers], *db[kMaxPackLayers];
+  int64_t packed[kMaxPackLayers];
   int32_t out[kMaxPackLayers], in[kMaxPackLayers];
   int32_t row0[kMaxPackLayers + 1];  // first global row of each layer
 };
@@ -37,7 +40,7 @@ __device__ __forceinline__ int layer_of(const PackLayers& L, int row) {
 }
 
 __global__ void __launch_bounds__(256)
-mlp_pack_fwd_kernel(const float* __restrict__ flat, PackLayers L, float* __restrict__ packed,
+mlp_pack_fwd_kernel(PackLayers L, float* __restrict__ packed,
                     const float* __restrict__ variance, float* __restrict__ inv_s) {
   const int lane = threadIdx.x & 63;
   const int row = blockIdx.x * 4 + (__builtin_amdgcn_readfirstlane(threadIdx.x) >> 6);
@@ -45,23 +48,28 @@ mlp_pack_fwd_kernel(const float* __restrict__ flat, PackLayers L, float* __restr
     *inv_s = fminf(fmaxf(expf(*variance * 10.f), 1e-6f), 1e6f);
   if (row >= L.row0[L.n]) return;
   const int l = layer_of(L, row), r = row - L.row0[l], in = L.in[l];
-  const float* v = flat + L.v[l] + (int64_t)r * in;
+  const float* v = L.v[l] + (int64_t)r * in;
   float* W = packed + L.packed[l] + (int64_t)r * in;
-  if (L.g[l] >= 0) {
+  if (L.g[l]) {
     float ss = 0.f;
     for (int i = lane; i < in; i += 64) ss += v[i] * v[i];
     const float nrm = sqrtf(wave_sum_f(ss));
-    const float g = flat[L.g[l] + r];
+    const float g = L.g[l][r];
     for (int i = lane; i < in; i += 64) W[i] = g * v[i] / nrm;
   } else {
     for (int i = lane; i < in; i += 64) W[i] = v[i];
   }
-  if (lane == 0) packed[L.packed[l] + (int64_t)L.out[l] * in + r] = flat[L.b[l] + r];
+  if (lane == 0) packed[L.packed[l] + (int64_t)L.out[l] * in + r] = L.b[l][r];
 }
 
+template <bool kAdd>
+__device__ __forceinline__ void put(float* p, float v) {
+  *p = kAdd ? *p + v : v;
+}
+
+template <bool kAdd>
 __global__ void __launch_bounds__(256)
-mlp_pack_bwd_kernel(const float* __restrict__ flat, PackLayers L,
-                    const float* __restrict__ g_packed, float* __restrict__ grad,
+mlp_pack_bwd_kernel(PackLayers L, const float* __restrict__ g_packed,
                     const float* __restrict__ variance, const float* __restrict__ g_inv_s,
                     float* __restrict__ g_variance) {
   const int lane = threadIdx.x & 63;
@@ -72,10 +80,10 @@ mlp_pack_bwd_kernel(const float* __restrict__ flat, PackLayers L,
   }
   if (row >= L.row0[L.n]) return;
   const int l = layer_of(L, row), r = row - L.row0[l], in = L.in[l];
-  const float* v = flat + L.v[l] + (int64_t)r * in;
+  const float* v = L.v[l] + (int64_t)r * in;
   const float* dW = g_packed + L.packed[l] + (int64_t)r * in;
-  float* dv = grad + L.v[l] + (int64_t)r * in;
-  if (L.g[l] >= 0) {
+  float* dv = L.dv[l] + (int64_t)r * in;
+  if (L.g[l]) {
     float ss = 0.f, dot = 0.f;
     for (int i = lane; i < in; i += 64) {
       ss += v[i] * v[i];
@@ -84,17 +92,21 @@ mlp_pack_bwd_kernel(const float* __restrict__ flat, PackLayers L,
     ss = wave_sum_f(ss);
     dot = wave_sum_f(dot);
     const float nrm = sqrtf(ss);
-    const float g = flat[L.g[l] + r];
+    const float g = L.g[l][r];
     const float a = g / nrm, c = dot / ss;
-    for (int i = lane; i < in; i += 64) dv[i] += a * (dW[i] - v[i] * c);
-    if (lane == 0) grad[L.g[l] + r] += dot / nrm;
+    for (int i = lane; i < in; i += 64) put<kAdd>(&dv[i], a * (dW[i] - v[i] * c));
+    if (lane == 0) put<kAdd>(&L.dg[l][r], dot / nrm);
   } else {
-    for (int i = lane; i < in; i += 64) dv[i] += dW[i];
+    for (int i = lane; i < in; i += 64) put<kAdd>(&dv[i], dW[i]);
   }
-  if (lane == 0) grad[L.b[l] + r] += g_packed[L.packed[l] + (int64_t)L.out[l] * in + r];
+  if (lane == 0)
+    put<kAdd>(&L.db[l][r], g_packed[L.packed[l] + (int64_t)L.out[l] * in + r]);
 }
 
-static int make_layers(const char* who, int32_t n_layers, const int64_t* desc, PackLayers* L) {
+// flat: the layers' tensors by offsets (gradients at the same offsets of grad);
+// else by addresses (gradients in grad, [dv | dg | db] per layer)
+static int make_layers(const char* who, int32_t n_layers, const int64_t* desc, const float* flat,
+                       float* grad, bool by_address, PackLayers* L) {
   SN_REQUIRE(n_layers > 0 && n_layers <= kMaxPackLayers, "%s: 1..%d layers", who,
              kMaxPackLayers);
   SN_REQUIRE(desc, "%s: null layer table", who);
@@ -104,9 +116,23 @@ static int make_layers(const char* who, int32_t n_layers, const int64_t* desc, P
     const int64_t* e = desc + 6 * l;  // v, g, b, packed, out, in
     SN_REQUIRE(e[0] >= 0 && e[2] >= 0 && e[3] >= 0 && e[4] > 0 && e[5] > 0,
                "%s: bad layer %d", who, l);
-    L->v[l] = e[0];
-    L->g[l] = e[1];
-    L->b[l] = e[2];
+    if (by_address) {
+      SN_REQUIRE(e[0] && e[2] && ((e[0] | e[1] | e[2]) & 3) == 0, "%s: bad layer %d", who, l);
+      L->v[l] = reinterpret_cast<const float*>(e[0]);
+      L->g[l] = reinterpret_cast<const float*>(e[1]);
+      L->b[l] = reinterpret_cast<const float*>(e[2]);
+      L->dv[l] = grad;
+      L->dg[l] = grad + e[4] * e[5];
+      L->db[l] = L->dg[l] + (e[1] ? e[4] : 0);
+      grad = L->db[l] + e[4];
+    } else {
+      L->v[l] = flat + e[0];
+      L->g[l] = e[1] >= 0 ? flat + e[1] : nullptr;
+      L->b[l] = flat + e[2];
+      L->dv[l] = grad + e[0];
+      L->dg[l] = grad + (e[1] >= 0 ? e[1] : 0);
+      L->db[l] = grad + e[2];
+    }
     L->packed[l] = e[3];
     L->out[l] = (int32_t)e[4];
     L->in[l] = (int32_t)e[5];
@@ -127,12 +153,12 @@ int sn_mlp_pack_fwd(const float* flat, int32_t n_layers, const int64_t* layers, 
                     const float* variance, float* inv_s, void* stream) {
   clear_error();
   PackLayers L;
-  int rc = make_layers("sn_mlp_pack_fwd", n_layers, layers, &L);
+  int rc = make_layers("sn_mlp_pack_fwd", n_layers, layers, flat, nullptr, false, &L);
   if (rc) return rc;
   SN_REQUIRE(flat && packed, "sn_mlp_pack_fwd: null pointer");
   const int rows = L.row0[L.n];
   mlp_pack_fwd_kernel<<<(unsigned)ceil_div(rows, 4), 256, 0, as_stream(stream)>>>(
-      flat, L, packed, variance, inv_s);
+      L, packed, variance, inv_s);
   return check_launch("sn_mlp_pack_fwd");
 }
 
@@ -141,13 +167,39 @@ int sn_mlp_pack_bwd(const float* flat, int32_t n_layers, const int64_t* layers,
                     const float* g_inv_s, float* g_variance, void* stream) {
   clear_error();
   PackLayers L;
-  int rc = make_layers("sn_mlp_pack_bwd", n_layers, layers, &L);
+  int rc = make_layers("sn_mlp_pack_bwd", n_layers, layers, flat, grad, false, &L);
   if (rc) return rc;
   SN_REQUIRE(flat && g_packed && grad, "sn_mlp_pack_bwd: null pointer");
   const int rows = L.row0[L.n];
-  mlp_pack_bwd_kernel<<<(unsigned)ceil_div(rows, 4), 256, 0, as_stream(stream)>>>(
-      flat, L, g_packed, grad, variance, g_inv_s, g_variance);
+  mlp_pack_bwd_kernel<true><<<(unsigned)ceil_div(rows, 4), 256, 0, as_stream(stream)>>>(
+      L, g_packed, variance, g_inv_s, g_variance);
   return check_launch("sn_mlp_pack_bwd");
+}
+
+int sn_mlp_pack_tensors_fwd(int32_t n_layers, const int64_t* layers, float* packed,
+                            void* stream) {
+  clear_error();
+  PackLayers L;
+  int rc = make_layers("sn_mlp_pack_tensors_fwd", n_layers, layers, nullptr, nullptr, true, &L);
+  if (rc) return rc;
+  SN_REQUIRE(packed, "sn_mlp_pack_tensors_fwd: null pointer");
+  const int rows = L.row0[L.n];
+  mlp_pack_fwd_kernel<<<(unsigned)ceil_div(rows, 4), 256, 0, as_stream(stream)>>>(
+      L, packed, nullptr, nullptr);
+  return check_launch("sn_mlp_pack_tensors_fwd");
+}
+
+int sn_mlp_pack_tensors_bwd(int32_t n_layers, const int64_t* layers, const float* g_packed,
+                            float* grad, void* stream) {
+  clear_error();
+  PackLayers L;
+  int rc = make_layers("sn_mlp_pack_tensors_bwd", n_layers, layers, nullptr, grad, true, &L);
+  if (rc) return rc;
+  SN_REQUIRE(g_packed && grad, "sn_mlp_pack_tensors_bwd: null pointer");
+  const int rows = L.row0[L.n];
+  mlp_pack_bwd_kernel<false><<<(unsigned)ceil_div(rows, 4), 256, 0, as_stream(stream)>>>(
+      L, g_packed, nullptr, nullptr, nullptr);
+  return check_launch("sn_mlp_pack_tensors_bwd");
 }
 
 }  // extern "C"

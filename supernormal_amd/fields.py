@@ -142,8 +142,8 @@ class SDFNetwork(nn.Module):
                          precision=getattr(self, "mlp_precision", "fp32"))
 
     def packed_mlp(self):
-        from .sdf import pack_mlp
-        return pack_mlp(self.mlp_layers())
+        from .sdf import pack_weight_norm
+        return pack_weight_norm(self._mlp_params())
 
     def fused_sdf(self, x):
         """sdf [N] via hash encode + MFMA MLP kernels (same values as sdf(x)[:, 0])."""
@@ -158,18 +158,16 @@ class SDFNetwork(nn.Module):
                                 self.active_levels())
 
     # -- folded MLP weights (used by the fused kernels) ----------------------
+    def _mlp_params(self):
+        """[(v or weight [out,in], g [out,1] or None, b [out])]"""
+        lins = [getattr(self, "lin" + str(l)) for l in range(0, self.num_layers - 1)]
+        return [(lin.weight_v, lin.weight_g, lin.bias) if self.weight_norm
+                else (lin.weight, None, lin.bias) for lin in lins]
+
     def mlp_layers(self):
         """[(W [out,in], b [out])] with weight norm applied (differentiable)."""
-        out = []
-        for l in range(0, self.num_layers - 1):
-            lin = getattr(self, "lin" + str(l))
-            if self.weight_norm:
-                v, g = lin.weight_v, lin.weight_g
-                W = g * v / v.norm(dim=1, keepdim=True)
-            else:
-                W = lin.weight
-            out.append((W, lin.bias))
-        return out
+        from .sdf import fold_weight_norm
+        return [(fold_weight_norm(v, g), b) for v, g, b in self._mlp_params()]
 
 
 class SingleVarianceNetwork(nn.Module):
