@@ -737,10 +737,11 @@ constexpr int kRedCols = 64, kRedGroups = 16;
 __global__ void __launch_bounds__(kRedCols * kRedGroups)
 reduce_rows_kernel(const float* __restrict__ partials, int64_t rows, int cols, float* __restrict__ out,
                    int accumulate) {
-  __shared__ float part[kRedGroups][kRedCols];
+  // (in 64 bits: a bias or norm gradient may be a sum that all but cancels)
+  __shared__ double part[kRedGroups][kRedCols];
   const int cl = threadIdx.x % kRedCols, g = threadIdx.x / kRedCols;
   const int c = blockIdx.x * kRedCols + cl;
-  float s = 0.f;
+  double s = 0.;
   if (c < cols) {
 #pragma unroll 8
     for (int64_t r = g; r < rows; r += kRedGroups) s += partials[r * cols + c];
@@ -748,10 +749,10 @@ reduce_rows_kernel(const float* __restrict__ partials, int64_t rows, int cols, f
   part[g][cl] = s;
   __syncthreads();
   if (g == 0 && c < cols) {
-    float t = 0.f;
+    double t = 0.;
 #pragma unroll
     for (int k = 0; k < kRedGroups; ++k) t += part[k][cl];
-    out[c] = accumulate ? out[c] + t : t;
+    out[c] = accumulate ? out[c] + (float)t : (float)t;
   }
 }
 

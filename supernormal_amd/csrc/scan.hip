@@ -221,16 +221,31 @@ int scan_flags_dev(const uint8_t* flags, int64_t n_cap, const int32_t* n_dev, in
                         s, "scan_flags_dev");
 }
 
+// Samples come sorted by ray: a wavefront's lanes are runs of equal indices,
+// whose first lane adds the run's length (a lane an atomic: 131 k samples of
+// 2048 rays 56 us, 4.5 so: atomics on one word are served one after another).
+// An index out of range counts as a run of -1.
 __global__ void count_indices_kernel(const int64_t* idx, int64_t n_cap, const int32_t* n_dev,
                                      int32_t n_rays, int32_t* counts, int32_t* n_bad) {
   const int64_t n = eff_n(n_cap, n_dev);
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * blockDim.x) {
-    int64_t r = idx[i];
-    if (r >= 0 && r < n_rays)
-      atomicAdd(&counts[r], 1);
-    else if (n_bad)
-      atomicAdd(n_bad, 1);
+  const int lane = threadIdx.x & 63;
+  // (the lanes of a wavefront stay together: 256 threads, a stride of whole blocks)
+  for (int64_t i0 = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i0 - lane < n;
+       i0 += (int64_t)gridDim.x * blockDim.x) {
+    const bool act = i0 < n;
+    const int64_t v = act ? idx[i0] : 0;
+    const int32_t r = v >= 0 && v < n_rays ? (int32_t)v : -1;
+    const int32_t before = __shfl_up(r, 1, 64);
+    const uint64_t heads = __ballot(act && (lane == 0 || r != before));
+    const int32_t n_act = __popcll(__ballot(act));
+    if (act && ((heads >> lane) & 1ull)) {
+      const uint64_t later = lane == 63 ? 0ull : heads >> (lane + 1);
+      const int32_t len = later ? __ffsll((unsigned long long)later) : n_act - lane;
+      if (r >= 0)
+        atomicAdd(&counts[r], len);
+      else if (n_bad)
+        atomicAdd(n_bad, len);
+    }
   }
 }
 

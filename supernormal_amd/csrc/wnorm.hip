@@ -27,7 +27,8 @@ struct PackLayers {
   int32_t row0[kMaxPackLayers + 1];  // first global row of each layer
 };
 
-__device__ __forceinline__ float wave_sum_f(float v) {
+template <typename T>
+__device__ __forceinline__ T wave_sum_f(T v) {
 #pragma unroll
   for (int off = 32; off >= 1; off >>= 1) v += __shfl_xor(v, off, 64);
   return v;
@@ -84,13 +85,13 @@ mlp_pack_bwd_kernel(PackLayers L, const float* __restrict__ g_packed,
   const float* dW = g_packed + L.packed[l] + (int64_t)r * in;
   float* dv = L.dv[l] + (int64_t)r * in;
   if (L.g[l]) {
-    float ss = 0.f, dot = 0.f;
+    // (in 64 bits: dL/dg of a row is a sum that cancels)
+    double ss2 = 0., dot2 = 0.;
     for (int i = lane; i < in; i += 64) {
-      ss += v[i] * v[i];
-      dot += dW[i] * v[i];
+      ss2 += (double)v[i] * v[i];
+      dot2 += (double)dW[i] * v[i];
     }
-    ss = wave_sum_f(ss);
-    dot = wave_sum_f(dot);
+    const float ss = (float)wave_sum_f(ss2), dot = (float)wave_sum_f(dot2);
     const float nrm = sqrtf(ss);
     const float g = L.g[l][r];
     const float a = g / nrm, c = dot / ss;

@@ -242,8 +242,8 @@ class _SDFGradFn(torch.autograd.Function):
         v = g_grad.contiguous()
         hargs = cfg.hash_args(ctx.n_active)
         encd = torch.empty((n, cfg.E), dtype=torch.float32, device=dev)
-        call("sn_hashgrid_bwd_bwd", ptr(x), n, ptr(params), *hargs, None, ptr(v), ptr(encd),
-             None, None, s)
+        call("sn_hashgrid_tangent_dev", ptr(x), n, None, ptr(params), None, *hargs, None, ptr(v),
+             ptr(encd), s)
         ge = torch.empty((n, cfg.E), dtype=torch.float32, device=dev)
         ged = torch.empty((n, cfg.E), dtype=torch.float32, device=dev)
         ws = workspace(lib.sn_mlp_bwd_workspace_bytes(n, cfg.E, cfg.d_hidden, cfg.n_layers, 1),
