@@ -4,9 +4,13 @@
 // graphs).
 //
 // Scan layout: a workgroup of 256 lanes owns a tile of 1024 consecutive
-// items (4 per lane); pass 1 writes one total per tile, pass 2 scans the tile
-// totals in one workgroup, pass 3 rescans each tile and adds its offset.  All
-// integer, so the result is exact and independent of the launch shape.
+// items (4 per lane); pass 1 writes one total per tile, pass 2 rescans each
+// tile behind the sum of the totals before it.  Above kDirectTiles tiles, whose
+// totals every workgroup would read, a workgroup between the two scans the
+// totals.  (A training iteration holds four scans of some 100 k items; a
+// kernel of that size is its launch, 4.5 us, so each pass counts: three
+// kernels and the flags' own were 18 us a scan, two are 9.)  All integer, so
+// the result is exact and independent of the launch shape.
 //
 // Every kernel takes a capacity n_cap (which sizes the launch) and an
 // optional device count n_dev (the number of valid items, <= n_cap), so the
@@ -18,6 +22,7 @@ namespace sn {
 constexpr int kScanBlock = 256;
 constexpr int kScanItems = 4;
 constexpr int kScanTile = kScanBlock * kScanItems;
+constexpr int64_t kDirectTiles = 2048;
 
 __device__ __forceinline__ int64_t eff_n(int64_t n_cap, const int32_t* n_dev) {
   if (!n_dev) return n_cap;
@@ -102,6 +107,16 @@ struct U8Src {
   const uint8_t* p;
   __device__ int32_t operator()(int64_t i) const { return p[i] ? 1 : 0; }
 };
+// whether a sample's end is not the next sample's start on its ray
+struct DiffSrc {
+  const int64_t* ri;
+  const float *t0, *t1;
+  int64_t n_cap;
+  const int32_t* n_dev;
+  __device__ int32_t operator()(int64_t i) const {
+    return i + 1 < eff_n(n_cap, n_dev) && ri[i + 1] == ri[i] && t1[i] == t0[i + 1] ? 0 : 1;
+  }
+};
 
 template <typename Src>
 __global__ void __launch_bounds__(kScanBlock)
@@ -167,11 +182,41 @@ struct FlagOffsetDst {
   __device__ void operator()(int64_t i, int32_t excl, int32_t v) const { p[i] = v ? excl : -1; }
 };
 
-template <typename Src, typename Dst>
+// the offset, and the sample itself to it when kept
+struct CompactDst {
+  int32_t* offs;
+  const int64_t* ri;
+  const float *t0, *t1;
+  int64_t* o_ri;
+  float *o_t0, *o_t1;
+  __device__ void operator()(int64_t i, int32_t excl, int32_t v) const {
+    offs[i] = excl;
+    if (v) {
+      o_ri[excl] = ri[i];
+      o_t0[excl] = t0[i];
+      o_t1[excl] = t1[i];
+    }
+  }
+};
+
+// kDirect: tiles holds the tiles' totals, and the last workgroup writes their
+// sum; else their scan.
+template <typename Src, typename Dst, bool kDirect>
 __global__ void __launch_bounds__(kScanBlock)
-tile_scan_write_kernel(Src src, int64_t n_cap, const int32_t* n_dev, const int32_t* tile_off,
-                       Dst dst) {
+tile_scan_write_kernel(Src src, int64_t n_cap, const int32_t* n_dev, const int32_t* tiles,
+                       int32_t* total_out, Dst dst) {
   const int64_t n = eff_n(n_cap, n_dev);
+  int32_t before = 0;
+  if constexpr (kDirect) {
+    const bool last = blockIdx.x == gridDim.x - 1;
+    if ((int64_t)blockIdx.x * kScanTile >= n && !last) return;  // uniform
+    int32_t part = 0;
+    for (uint32_t t = threadIdx.x; t < blockIdx.x; t += kScanBlock) part += tiles[t];
+    block_excl_scan(part, &before);
+    if (last && total_out && threadIdx.x == 0) *total_out = before + tiles[blockIdx.x];
+  } else {
+    before = tiles[blockIdx.x];
+  }
   const int64_t base = (int64_t)blockIdx.x * kScanTile + threadIdx.x * kScanItems;
   int32_t v[kScanItems];
   int32_t s = 0;
@@ -181,7 +226,7 @@ tile_scan_write_kernel(Src src, int64_t n_cap, const int32_t* n_dev, const int32
     s += v[j];
   }
   int32_t tot;
-  int32_t off = block_excl_scan(s, &tot) + tile_off[blockIdx.x];
+  int32_t off = block_excl_scan(s, &tot) + before;
 #pragma unroll
   for (int j = 0; j < kScanItems; ++j) {
     if (base + j < n) dst(base + j, off, v[j]);
@@ -208,17 +253,25 @@ int exclusive_scan(Src src, int64_t n_cap, const int32_t* n_dev, Dst dst, int32_
   }
   const int64_t n_tiles = ceil_div(n_cap, kScanTile);
   tile_totals_kernel<<<(unsigned)n_tiles, kScanBlock, 0, s>>>(src, n_cap, n_dev, tiles);
-  scan_tiles_kernel<<<1, kScanBlock, 0, s>>>(tiles, n_cap, n_dev, total);
-  tile_scan_write_kernel<<<(unsigned)n_tiles, kScanBlock, 0, s>>>(src, n_cap, n_dev, tiles, dst);
+  if (n_tiles <= kDirectTiles) {
+    tile_scan_write_kernel<Src, Dst, true><<<(unsigned)n_tiles, kScanBlock, 0, s>>>(
+        src, n_cap, n_dev, tiles, total, dst);
+  } else {
+    scan_tiles_kernel<<<1, kScanBlock, 0, s>>>(tiles, n_cap, n_dev, total);
+    tile_scan_write_kernel<Src, Dst, false><<<(unsigned)n_tiles, kScanBlock, 0, s>>>(
+        src, n_cap, n_dev, tiles, nullptr, dst);
+  }
   return check_launch(what);
 }
 
-// offsets[i] = number of flagged items before i when flags[i] != 0, else -1;
-// *total = number of flagged items (device).  Used by the sync-free iteration.
-int scan_flags_dev(const uint8_t* flags, int64_t n_cap, const int32_t* n_dev, int32_t* offsets,
-                   int32_t* total, void* ws, size_t ws_bytes, hipStream_t s) {
-  return exclusive_scan(U8Src{flags}, n_cap, n_dev, FlagOffsetDst{offsets}, total, ws, ws_bytes,
-                        s, "scan_flags_dev");
+// offsets[i] = number of samples before i whose end is not the next sample's
+// start when i's is not, else -1; *total = number of such samples (device).
+// Used by the sync-free iteration.
+int scan_diff_dev(const int64_t* ri, const float* t0, const float* t1, int64_t n_cap,
+                  const int32_t* n_dev, int32_t* offsets, int32_t* total, void* ws,
+                  size_t ws_bytes, hipStream_t s) {
+  return exclusive_scan(DiffSrc{ri, t0, t1, n_cap, n_dev}, n_cap, n_dev, FlagOffsetDst{offsets},
+                        total, ws, ws_bytes, s, "scan_diff_dev");
 }
 
 // Samples come sorted by ray: a wavefront's lanes are runs of equal indices,
@@ -245,21 +298,6 @@ __global__ void count_indices_kernel(const int64_t* idx, int64_t n_cap, const in
         atomicAdd(&counts[r], len);
       else if (n_bad)
         atomicAdd(n_bad, len);
-    }
-  }
-}
-
-__global__ void compact_kernel(const uint8_t* keep, int64_t n_cap, const int32_t* n_dev,
-                               const int32_t* offs, const int64_t* ri, const float* t0,
-                               const float* t1, int64_t* o_ri, float* o_t0, float* o_t1) {
-  const int64_t n = eff_n(n_cap, n_dev);
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * blockDim.x) {
-    if (keep[i]) {
-      int32_t o = offs[i];
-      o_ri[o] = ri[i];
-      o_t0[o] = t0[i];
-      o_t1[o] = t1[i];
     }
   }
 }
@@ -377,12 +415,11 @@ int sn_compact_samples_dev(const uint8_t* keep, int32_t n_cap, const int32_t* n_
   hipStream_t s = as_stream(stream);
   int32_t* offs = reinterpret_cast<int32_t*>(ws);
   size_t obytes = align_up((size_t)(n_cap > 0 ? n_cap : 1) * sizeof(int32_t), 256);
-  int rc = exclusive_scan(U8Src{keep}, n_cap, n_dev, OffsetDst{offs}, n_out,
-                          (char*)ws + obytes, ws_bytes - obytes, s, "sn_compact_samples/scan");
+  int rc = exclusive_scan(U8Src{keep}, n_cap, n_dev,
+                          CompactDst{offs, ray_indices, t_starts, t_ends, out_ray_indices,
+                                     out_t_starts, out_t_ends},
+                          n_out, (char*)ws + obytes, ws_bytes - obytes, s, "sn_compact_samples");
   if (rc || n_cap == 0) return rc;
-  compact_kernel<<<grid_for(n_cap, 256), 256, 0, s>>>(keep, n_cap, n_dev, offs, ray_indices,
-                                                      t_starts, t_ends, out_ray_indices,
-                                                      out_t_starts, out_t_ends);
   if (packed_in && packed_out && n_rays > 0)
     compact_packed_kernel<<<(unsigned)ceil_div(n_rays, 256), 256, 0, s>>>(
         packed_in, n_rays, n_cap, n_dev, offs, n_out, packed_out);

@@ -45,8 +45,9 @@ inline unsigned grid_for(int64_t n, int block, int64_t max_blocks = 256 * 16) {
 size_t scan_ws_bytes(int64_t n);
 int fill_i32(int32_t* p, int64_t n, int32_t v, hipStream_t s);
 int fill_f32(float* p, int64_t n, float v, hipStream_t s);
-int scan_flags_dev(const uint8_t* flags, int64_t n_cap, const int32_t* n_dev, int32_t* offsets,
-                   int32_t* total, void* ws, size_t ws_bytes, hipStream_t s);
+int scan_diff_dev(const int64_t* ri, const float* t0, const float* t1, int64_t n_cap,
+                  const int32_t* n_dev, int32_t* offsets, int32_t* total, void* ws,
+                  size_t ws_bytes, hipStream_t s);
 
 // mlp.hip: out[c] (+)= sum over rows of part[row][c], fixed order
 int mlp_reduce_rows(const float* part, int64_t rows, int cols, float* out, int accumulate,

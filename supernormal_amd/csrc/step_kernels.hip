@@ -22,19 +22,6 @@
 namespace sn {
 
 __global__ void __launch_bounds__(256)
-diff_flags_kernel(const int64_t* __restrict__ ri, const float* __restrict__ t0,
-                  const float* __restrict__ t1, int64_t n_cap, const int32_t* __restrict__ n_dev,
-                  uint8_t* __restrict__ flags) {
-  const int64_t n = dev_count(n_cap, n_dev);
-  for (int64_t s = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; s < n;
-       s += (int64_t)gridDim.x * blockDim.x) {
-    bool d = true;
-    if (s + 1 < n) d = !(ri[s + 1] == ri[s] && t1[s] == t0[s + 1]);
-    flags[s] = d ? 1 : 0;
-  }
-}
-
-__global__ void __launch_bounds__(256)
 centre_points_kernel(const int64_t* __restrict__ ri, const float* __restrict__ t0,
                      const float* __restrict__ t1, int64_t n_cap,
                      const int32_t* __restrict__ n_dev, const float* __restrict__ o_c,
@@ -158,7 +145,6 @@ occ_sample_kernel(const int64_t* __restrict__ occ_list, const int32_t* __restric
   }
 }
 
-static size_t flags_bytes(int64_t n) { return align_up((size_t)(n > 0 ? n : 1), 256); }
 
 }  // namespace sn
 
@@ -167,7 +153,7 @@ using namespace sn;
 extern "C" {
 
 size_t sn_step_workspace_bytes(int64_t n_cap) {
-  return flags_bytes(n_cap) + align_up(sizeof(int32_t) * 4, 256) + scan_ws_bytes(n_cap);
+  return scan_ws_bytes(n_cap);
 }
 
 int sn_centre_points(const int64_t* ray_indices, const float* t_starts, const float* t_ends,
@@ -187,12 +173,8 @@ int sn_centre_points(const int64_t* ray_indices, const float* t_starts, const fl
     int rc = fill_i32(n_diff, 1, 0, s);
     return rc ? rc : fill_i32(n_eval, 1, 0, s);
   }
-  uint8_t* flags = reinterpret_cast<uint8_t*>(ws);
-  char* rest = (char*)ws + flags_bytes(n_cap) + align_up(sizeof(int32_t) * 4, 256);
-  diff_flags_kernel<<<grid_for(n_cap, 256), 256, 0, s>>>(ray_indices, t_starts, t_ends, n_cap,
-                                                         n_dev, flags);
-  int rc = scan_flags_dev(flags, n_cap, n_dev, diff_idx, n_diff, rest,
-                          ws_bytes - (rest - (char*)ws), s);
+  int rc = scan_diff_dev(ray_indices, t_starts, t_ends, n_cap, n_dev, diff_idx, n_diff, ws,
+                         ws_bytes, s);
   if (rc) return rc;
   centre_points_kernel<<<grid_for(n_cap, 256), 256, 0, s>>>(
       ray_indices, t_starts, t_ends, n_cap, n_dev, rays_o_c, rays_d_c, centre_stride, diff_idx,
@@ -231,12 +213,8 @@ int sn_patch_points(const int64_t* ray_indices, const float* t_starts, const flo
     int rc = fill_i32(n_diff, 1, 0, s);
     return rc ? rc : fill_i32(n_eval, 1, 0, s);
   }
-  uint8_t* flags = reinterpret_cast<uint8_t*>(ws);
-  char* rest = (char*)ws + flags_bytes(n_cap) + align_up(sizeof(int32_t) * 4, 256);
-  diff_flags_kernel<<<grid_for(n_cap, 256), 256, 0, s>>>(ray_indices, t_starts, t_ends, n_cap,
-                                                         n_dev, flags);
-  int rc = scan_flags_dev(flags, n_cap, n_dev, diff_idx, n_diff, rest,
-                          ws_bytes - (rest - (char*)ws), s);
+  int rc = scan_diff_dev(ray_indices, t_starts, t_ends, n_cap, n_dev, diff_idx, n_diff, ws,
+                         ws_bytes, s);
   if (rc) return rc;
   const int32_t kc = (patch_h / 2) * patch_w + patch_w / 2;
   patch_points_kernel<<<grid_for(n_cap * P, 256), 256, 0, s>>>(
