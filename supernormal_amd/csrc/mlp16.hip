@@ -385,7 +385,7 @@ mlp16_fwd_kernel(const float* __restrict__ x, const float* __restrict__ enc, int
 // the network the sdf value comes from to the same resolution.
 // ---------------------------------------------------------------------------
 template <int H, int NH, int KB0>
-__global__ void __launch_bounds__(64 * kWaves)
+__global__ void __launch_bounds__(64 * kWaves, 4)  // 113 registers; unbounded 130, 3 wavefronts
 mlp16_fwd_grad_kernel(const float* __restrict__ x, const float* __restrict__ enc, int E, int vec4,
                       int64_t n_cap, const int32_t* __restrict__ n_dev,
                       const float* __restrict__ mlp, float beta, float* __restrict__ sdf_out,
